@@ -33,6 +33,8 @@
 // order, which makes every line access of every direction, and the sequential
 // accesses of phases A and C, free of bank conflicts for 32 and for 64 banks.
 #pragma once
+#include <type_traits>
+
 #include "dg_common.hpp"
 #include "indicator2d.hpp"
 
@@ -115,9 +117,10 @@ __device__ __forceinline__ int xcd_remap_block(int b, int nb) {
   return (x < r) ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
 }
 
+// (compiler vectors: an array of HIP's float4 structs stayed in scratch memory)
 template <int BYTES> struct ChunkOf;
-template <> struct ChunkOf<16> { using type = float4; };
-template <> struct ChunkOf<8> { using type = float2; };
+template <> struct ChunkOf<16> { typedef float type __attribute__((ext_vector_type(4))); };
+template <> struct ChunkOf<8> { typedef float type __attribute__((ext_vector_type(2))); };
 template <> struct ChunkOf<4> { using type = float; };
 
 // A full tile of EPB elements moves between global memory and LDS in chunks of
@@ -180,14 +183,15 @@ template <int VOL> struct VolTraits {
   static constexpr bool CONS = !RAN || HG;
 };
 
-// Per-lane line context: which line the lane owns and the four face states
-// (neighbour states loaded from global memory at kernel entry, own states read
-// from the staged tile) so that no load latency sits inside the line phase.
+// Per-lane line context: which line the lane owns and the two neighbour face
+// states, loaded from global memory at kernel entry so that no load latency sits
+// inside the line phase (the own face states are read from the staged tile where
+// the surface fluxes use them).
 template <typename T, int V> struct LineCtx {
   int el, line, base;
   bool valid;
   int fm, fp;  // BND variants: offsets of the given fluxes of mortar faces at the -O / +O face, or -1
-  T ul_m[V], ur_p[V], own0[V], own1[V];
+  T ul_m[V], ur_p[V];
 };
 
 // Line of this lane in direction o (wave-uniform, runtime) and the ids of the
@@ -275,64 +279,41 @@ __device__ __forceinline__ void line_loads(const ElemArgs<T> &a, LineCtx<T, D + 
   }
 }
 
-// own face states from the staged tile (AoS [q][v])
-template <typename T, int D, int N, int EPB, int O>
-__device__ __forceinline__ void line_own(const T *__restrict__ staged, LineCtx<T, D + 2> &c) {
+// LDS slots of the line's nodes
+template <int D, int N, int EPB, int O> __device__ __forceinline__ void line_slots(int q0, int *pq) {
   using LY = Layout<D, N, EPB>;
-  constexpr int n = N + 1, NN = LY::NN, V = D + 2;
-  constexpr int st = ipow_c(n, O);
-  if (!c.valid) return;
-  const int q0 = c.el * NN + c.base;
+  pq[0] = LY::phys(q0);
 #pragma unroll
-  for (int v = 0; v < V; ++v) {
-    c.own0[v] = staged[q0 * V + v];
-    c.own1[v] = staged[(q0 + (n - 1) * st) * V + v];
-  }
+  for (int i = 1; i < N + 1; ++i) pq[i] = LY::template phys_line<O>(pq[0], q0, i);
 }
 
-// One line of direction O: volume terms, the two surface terms, LDS write.
+// Surface terms of one line of direction O, added to acc. staged: the tile's
+// states [q][v]. With flux_ranocha and a representation of the node records
+// that holds the sound speed (FP64, and FP32 in the square-root
+// representation), the own face states' primitives and sound speeds come from
+// the records of the two end nodes: wend (read here in FP64).
+template <typename T, int D, int N> using LineRecord = std::conditional_t<sizeof(T) == 8, NodeD<D>, NodeR<T, D>>;
+
+template <int D, int SZ> __device__ __forceinline__ void load_record(NodeD<D> &x, const double *s_w, int q) {
+  x.r = s_w[0 * SZ + q];
+  x.t = s_w[1 * SZ + q];
+#pragma unroll
+  for (int d = 0; d < D; ++d) x.h[d] = s_w[(2 + d) * SZ + q];
+  x.hp = s_w[(2 + D) * SZ + q];
+}
+
 template <typename T, int D, int N, int VOL, int EPB, int O, bool BND>
-__device__ __forceinline__ void line_work(const ElemArgs<T> &a, const DGConst<T, N> &k, const LineCtx<T, D + 2> &c,
-                                          const T *__restrict__ s_w, const T *__restrict__ s_c,
-                                          T *__restrict__ s_d, const double *__restrict__ s_alpha) {
+__device__ __forceinline__ void line_faces(const ElemArgs<T> &a, const DGConst<T, N> &k, const LineCtx<T, D + 2> &c,
+                                           const T *__restrict__ staged, const T *__restrict__ s_w,
+                                           LineRecord<T, D, N> (&wend)[2], T (&acc)[N + 1][D + 2]) {
   using LY = Layout<D, N, EPB>;
   using VT = VolTraits<VOL>;
   constexpr int n = N + 1, NN = LY::NN, V = D + 2, SZ = LY::SIZE;
   constexpr int st = ipow_c(n, O);
-  if (!c.valid) return;
-  const int el = c.el;
-  const int q0 = el * NN + c.base;
-  const T gamma = a.gamma;
-  const T gm1 = gamma - T(1);
-  const T igm1 = a.inv_gamma_m1;
-  // node records in the square-root representation (FP32, polydeg <= 3); the
-  // own face states' primitives and sound speeds then come from the records of
-  // the two end nodes
-  constexpr bool SQ = node_sqrt_rep<T, N>();
-  constexpr bool OWN_FROM_W = VT::RAN && SQ;
-  NodeR<T, D> wend[2];
-
-  int pq[n];
-  pq[0] = LY::phys(q0);
-#pragma unroll
-  for (int i = 1; i < n; ++i) pq[i] = LY::template phys_line<O>(pq[0], q0, i);
-
-  T acc[n][V];
-#pragma unroll
-  for (int i = 0; i < n; ++i)
-#pragma unroll
-    for (int v = 0; v < V; ++v) acc[i][v] = T(0);
-
-  double alpha = 0.0;
-  bool blend = false;
-  if constexpr (VT::HG) {
-    alpha = s_alpha[el];
-    const double atol = sizeof(T) == 8 ? 1.8189894035458565e-12 : 1.1920928955078125e-5;
-    blend = !(alpha <= atol && alpha >= -atol);
-  }
-
-  // ---------------- interface fluxes + surface integral ----------------
-  // (evaluated after the volume integral, see the end of this function)
+  constexpr bool F64 = sizeof(T) == 8;
+  constexpr bool OWN_FROM_W = VT::RAN && (node_sqrt_rep<T, N>() || F64);
+  const int q0 = c.el * NN + c.base;
+  const T gamma = a.gamma, gm1 = gamma - T(1);
   const T factor = k.inv_w[0];  // inverse_weights[1] of the reference
   // mortar faces (BND variants): the flux computed by mortar_flux_kernel
   auto given_flux = [&](int off, T *F) {
@@ -343,54 +324,92 @@ __device__ __forceinline__ void line_work(const ElemArgs<T> &a, const DGConst<T,
       }
     }
   };
-  auto faces = [&]() {
-    T F[V];
-    bool done = false;
-    if constexpr (OWN_FROM_W) {
-      if (a.surface_flux == FLUX_LLF || a.surface_flux == FLUX_LLF_NAIVE) {
-        const bool naive = a.surface_flux == FLUX_LLF_NAIVE;
-        ConsP<T, D> own_face[2];
-        T own_c[2];
-        consp_from_node<D>(c.own0, wend[0], a.sqrt_gamma, own_face[0], own_c[0]);
-        consp_from_node<D>(c.own1, wend[1], a.sqrt_gamma, own_face[1], own_c[1]);
-        // twice the LLF flux with half the weight (bitwise the same terms);
-        // a given mortar flux is doubled to match
-        const T hfactor = T(0.5) * factor;
-        auto given_flux2 = [&](int off, T *F2) {
-          if constexpr (BND) {
-            if (off >= 0) {
+  T F[V], own0[V], own1[V];
 #pragma unroll
-              for (int v = 0; v < V; ++v) F2[v] = T(2) * a.mflux[off + v];
-            }
-          }
-        };
-        ConsP<T, D> nb;
-        consp_from_cons<T, D>(c.ul_m, gm1, nb);  // -O face: element is the right state
-        flux_llf_pc2<T, D, O>(nb, own_face[0], Prec<T>::sqrt_(gamma * nb.p * nb.irho), own_c[0], naive, F);
-        given_flux2(c.fm, F);
-#pragma unroll
-        for (int v = 0; v < V; ++v) acc[0][v] = tfma(-F[v], hfactor, acc[0][v]);
-        consp_from_cons<T, D>(c.ur_p, gm1, nb);  // +O face: element is the left state
-        flux_llf_pc2<T, D, O>(own_face[1], nb, own_c[1], Prec<T>::sqrt_(gamma * nb.p * nb.irho), naive, F);
-        given_flux2(c.fp, F);
-#pragma unroll
-        for (int v = 0; v < V; ++v) acc[n - 1][v] = tfma(F[v], hfactor, acc[n - 1][v]);
-        done = true;
+  for (int v = 0; v < V; ++v) {
+    own0[v] = staged[q0 * V + v];
+    own1[v] = staged[(q0 + (n - 1) * st) * V + v];
+  }
+  bool done = false;
+  if constexpr (OWN_FROM_W) {
+    if (a.surface_flux == FLUX_LLF || a.surface_flux == FLUX_LLF_NAIVE) {
+      const bool naive = a.surface_flux == FLUX_LLF_NAIVE;
+      ConsP<T, D> own_face[2];
+      T own_c[2];
+      if constexpr (F64) {
+        load_record<D, SZ>(wend[0], s_w, LY::phys(q0));
+        load_record<D, SZ>(wend[1], s_w, LY::phys(q0 + (n - 1) * st));
       }
-    }
-    if (!done) {
-      num_flux_c<T, D, O, VOL == VOL_PURE_FV>(a.surface_flux, c.ul_m, c.own0, gamma, F);  // -O face: element is the right state
-      given_flux(c.fm, F);
+      consp_from_node<D>(own0, wend[0], a.sqrt_gamma, own_face[0], own_c[0]);
+      consp_from_node<D>(own1, wend[1], a.sqrt_gamma, own_face[1], own_c[1]);
+      // twice the LLF flux with half the weight (bitwise the same terms);
+      // a given mortar flux is doubled to match
+      const T hfactor = T(0.5) * factor;
+      auto given_flux2 = [&](int off, T *F2) {
+        if constexpr (BND) {
+          if (off >= 0) {
 #pragma unroll
-      for (int v = 0; v < V; ++v) acc[0][v] = tfma(-F[v], factor, acc[0][v]);
-      num_flux_c<T, D, O, VOL == VOL_PURE_FV>(a.surface_flux, c.own1, c.ur_p, gamma, F);  // +O face: element is the left state
-      given_flux(c.fp, F);
+            for (int v = 0; v < V; ++v) F2[v] = T(2) * a.mflux[off + v];
+          }
+        }
+      };
+      ConsP<T, D> nb;
+      consp_from_cons<T, D>(c.ul_m, gm1, nb);  // -O face: element is the right state
+      flux_llf_pc2<T, D, O>(nb, own_face[0], Prec<T>::sqrt_(gamma * nb.p * nb.irho), own_c[0], naive, F);
+      given_flux2(c.fm, F);
 #pragma unroll
-      for (int v = 0; v < V; ++v) acc[n - 1][v] = tfma(F[v], factor, acc[n - 1][v]);
+      for (int v = 0; v < V; ++v) acc[0][v] = tfma(-F[v], hfactor, acc[0][v]);
+      consp_from_cons<T, D>(c.ur_p, gm1, nb);  // +O face: element is the left state
+      flux_llf_pc2<T, D, O>(own_face[1], nb, own_c[1], Prec<T>::sqrt_(gamma * nb.p * nb.irho), naive, F);
+      given_flux2(c.fp, F);
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[n - 1][v] = tfma(F[v], hfactor, acc[n - 1][v]);
+      done = true;
     }
-  };
+  }
+  if (!done) {
+    num_flux_c<T, D, O, VOL == VOL_PURE_FV>(a.surface_flux, c.ul_m, own0, gamma, F);  // -O face: element is the right state
+    given_flux(c.fm, F);
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[0][v] = tfma(-F[v], factor, acc[0][v]);
+    num_flux_c<T, D, O, VOL == VOL_PURE_FV>(a.surface_flux, own1, c.ur_p, gamma, F);  // +O face: element is the left state
+    given_flux(c.fp, F);
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[n - 1][v] = tfma(F[v], factor, acc[n - 1][v]);
+  }
+}
 
-  // ---------------- volume integral ----------------
+// One line of direction O: volume terms added to acc. s_w, s_c: node records
+// and conservative states by variable; s_l: this lane's slots for logarithms
+// (FP64 flux_ranocha), NT apart. wend receives the records of the two end nodes
+// (FP32 flux_ranocha), pq the slots of the line's nodes.
+template <typename T, int D, int N, int VOL, int EPB, int NT, int O>
+__device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<T, N> &k, const LineCtx<T, D + 2> &c,
+                                            const T *__restrict__ s_w, const T *__restrict__ s_c,
+                                            const double *__restrict__ s_alpha, T *__restrict__ s_l,
+                                            LineRecord<T, D, N> (&wend)[2], int (&pq)[N + 1],
+                                            T (&acc)[N + 1][D + 2]) {
+  using LY = Layout<D, N, EPB>;
+  using VT = VolTraits<VOL>;
+  constexpr int n = N + 1, NN = LY::NN, V = D + 2, SZ = LY::SIZE;
+  constexpr bool F64 = sizeof(T) == 8;
+  const int el = c.el;
+  const int q0 = el * NN + c.base;
+  const T gamma = a.gamma;
+  const T gm1 = gamma - T(1);
+  const T igm1 = a.inv_gamma_m1;
+  constexpr bool SQ = node_sqrt_rep<T, N>();
+  constexpr bool KEEP_ENDS = VT::RAN && SQ;
+  line_slots<D, N, EPB, O>(q0, pq);
+
+  double alpha = 0.0;
+  bool blend = false;
+  if constexpr (VT::HG) {
+    alpha = s_alpha[el];
+    const double atol = sizeof(T) == 8 ? 1.8189894035458565e-12 : 1.1920928955078125e-5;
+    blend = !(alpha <= atol && alpha >= -atol);
+  }
+
   if constexpr (VOL == VOL_WEAK) {
 #pragma unroll
     for (int b = 0; b < n; ++b) {
@@ -409,7 +428,113 @@ __device__ __forceinline__ void line_work(const ElemArgs<T> &a, const DGConst<T,
       }
     }
   }
-  if constexpr (VT::RAN) {
+  if constexpr (VT::RAN && F64) {
+    const T higm1 = T(0.5) * igm1;
+    auto add_pair = [&](int i, int j, const T *f) {
+      const T di = k.Dsplit[i * n + j], dj = k.Dsplit[j * n + i];
+#pragma unroll
+      for (int v = 0; v < V - 1; ++v) {
+        acc[i][v] = tfma(di, f[v], acc[i][v]);
+        acc[j][v] = tfma(dj, f[v], acc[j][v]);
+      }
+      acc[i][V - 1] = tfma(k.Dsplit2[i * n + j], f[V - 1], acc[i][V - 1]);
+      acc[j][V - 1] = tfma(k.Dsplit2[j * n + i], f[V - 1], acc[j][V - 1]);
+    };
+    // Which form of the means the line takes. It depends on this line alone, so
+    // that results do not depend on the tile; the wavefront takes the cheapest
+    // path that serves all its lines. The high words h of two positive doubles
+    // order them, and their quotient is at most 1 + (h1 - h0) 2^-20 (the high word
+    // grows linearly within a binade, so per factor slowest at its start). So the
+    // largest minus the smallest high word of the line's roots bounds every
+    // pair's |f| = (quotient - 1) / (quotient + 1), in half the instructions of
+    // FP64 minima, maxima and products.
+    NodeD<D> w[n];
+#pragma unroll
+    for (int i = 0; i < n; ++i) load_record<D, SZ>(w[i], s_w, pq[i]);
+    uint32_t lo_r = high_word(w[0].r), hi_r = lo_r, lo_t = high_word(w[0].t), hi_t = lo_t;
+#pragma unroll
+    for (int i = 1; i < n; ++i) {
+      const uint32_t r = high_word(w[i].r), t = high_word(w[i].t);
+      lo_r = min(lo_r, r);
+      hi_r = max(hi_r, r);
+      lo_t = min(lo_t, t);
+      hi_t = max(hi_t, t);
+    }
+    const uint32_t sign = (hi_r | hi_t) & 0x80000000u;  // a negative value: logarithms, which give NaN
+    const uint32_t spread = max(max(hi_r - lo_r, hi_t - lo_t), sign);
+    auto fresh = [](const T *p) {
+      int z0 = 0;
+      asm volatile("" : "+v"(z0));
+      return p + z0;
+    };
+    const int kind = spread <= MeanSeriesShort::kMaxSpread  ? MEAN_SHORT
+                     : spread <= MeanSeriesLong::kMaxSpread ? MEAN_LONG
+                                                            : MEAN_LOG;
+    auto near_pairs = [&](const NodeD<D> (&x)[n]) {
+#pragma unroll
+      for (int i = 0; i < n; ++i)
+#pragma unroll
+        for (int j = i + 1; j < n; ++j) {
+          T f[V];
+          flux_ranocha_near<false, D, O>(x[i], x[j], kind, higm1, f);
+          add_pair(i, j, f);
+        }
+    };
+    if (__builtin_amdgcn_ballot_w64(kind != MEAN_SHORT) == 0) {
+      if constexpr (n <= 4) {
+        near_pairs(w);
+      } else {
+        // the records read again (the opaque zero offset keeps the copies apart):
+        // 141 us with, 153 us without (3D polydeg 4 RHS, 32^3 elements)
+        const T *sw = fresh(s_w);
+        NodeD<D> x[n];
+#pragma unroll
+        for (int i = 0; i < n; ++i) load_record<D, SZ>(x[i], sw, pq[i]);
+        near_pairs(x);
+      }
+    } else if (__builtin_amdgcn_ballot_w64(kind == MEAN_LOG) == 0) {
+      // each pair's records read again and the pairs kept in sequence (here and
+      // below): held or interleaved they would set the register allocation of
+      // the whole kernel
+#pragma unroll
+      for (int i = 0; i < n; ++i)
+#pragma unroll
+        for (int j = i + 1; j < n; ++j) {
+          T f[V];
+          const T *sw = fresh(s_w);
+          NodeD<D> wi, wj;
+          load_record<D, SZ>(wi, sw, pq[i]);
+          load_record<D, SZ>(wj, sw, pq[j]);
+          flux_ranocha_near<true, D, O>(wi, wj, kind, higm1, f);
+          add_pair(i, j, f);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    } else {
+      // Strong shocks: the logarithms of the line's roots, through LDS.
+#pragma unroll
+      for (int i = 0; i < n; ++i) {
+        const T *sw = fresh(s_w);
+        s_l[(2 * i) * NT] = Prec<T>::ln(sw[0 * SZ + pq[i]]);
+        s_l[(2 * i + 1) * NT] = Prec<T>::ln(sw[1 * SZ + pq[i]]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < n; ++i)
+#pragma unroll
+        for (int j = i + 1; j < n; ++j) {
+          T f[V];
+          const T *sw = fresh(s_w), *sl = fresh(s_l);
+          NodeD<D> wi, wj;
+          load_record<D, SZ>(wi, sw, pq[i]);
+          load_record<D, SZ>(wj, sw, pq[j]);
+          flux_ranocha_far<D, O>(wi, wj, kind, sl[(2 * i) * NT], sl[(2 * j) * NT], sl[(2 * i + 1) * NT],
+                                 sl[(2 * j + 1) * NT], higm1, f);
+          add_pair(i, j, f);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+  }
+  if constexpr (VT::RAN && !F64) {
     NodeR<T, D> w[n];
     auto load_w = [&](int i) {
       w[i].r = s_w[0 * SZ + pq[i]];
@@ -422,12 +547,12 @@ __device__ __forceinline__ void line_work(const ElemArgs<T> &a, const DGConst<T,
     };
 #pragma unroll
     for (int i = 0; i < n; ++i) load_w(i);
-    if constexpr (OWN_FROM_W) {  // the end records, for the faces after the volume terms
+    if constexpr (KEEP_ENDS) {  // the end records, for the faces after the volume terms
       wend[0] = w[0];
       wend[1] = w[n - 1];
     }
     bool fast = false;
-    if constexpr (sizeof(T) == 4) {
+    {
       // the division-free series applies when every log ratio on the line is in range
       T lo_r = w[0].lrho, hi_r = w[0].lrho, lo_b = w[0].lbeta, hi_b = w[0].lbeta;
 #pragma unroll
@@ -441,55 +566,49 @@ __device__ __forceinline__ void line_work(const ElemArgs<T> &a, const DGConst<T,
       fast = __builtin_amdgcn_ballot_w64(!in_range) == 0;  // wave-uniform
     }
     if (fast) {
-      if constexpr (sizeof(T) == 4) {
 #pragma unroll
-        for (int i = 0; i < n; ++i)
+      for (int i = 0; i < n; ++i)
 #pragma unroll
-          for (int j = i + 1; j < n; ++j) {
-            T f[V];
-            flux_ranocha_fast<D, O, SQ>(w[i], w[j], T(0.5) * igm1, f);
-            const T di = k.Dsplit[i * n + j], dj = k.Dsplit[j * n + i];
+        for (int j = i + 1; j < n; ++j) {
+          T f[V];
+          flux_ranocha_fast<D, O, SQ>(w[i], w[j], T(0.5) * igm1, f);
+          const T di = k.Dsplit[i * n + j], dj = k.Dsplit[j * n + i];
 #pragma unroll
-            for (int v = 0; v < V - 1; ++v) {
-              acc[i][v] = tfma(di, f[v], acc[i][v]);
-              acc[j][v] = tfma(dj, f[v], acc[j][v]);
-            }
-            acc[i][V - 1] = tfma(k.Dsplit2[i * n + j], f[V - 1], acc[i][V - 1]);
-            acc[j][V - 1] = tfma(k.Dsplit2[j * n + i], f[V - 1], acc[j][V - 1]);
+          for (int v = 0; v < V - 1; ++v) {
+            acc[i][v] = tfma(di, f[v], acc[i][v]);
+            acc[j][v] = tfma(dj, f[v], acc[j][v]);
           }
-      }
+          acc[i][V - 1] = tfma(k.Dsplit2[i * n + j], f[V - 1], acc[i][V - 1]);
+          acc[j][V - 1] = tfma(k.Dsplit2[j * n + i], f[V - 1], acc[j][V - 1]);
+        }
     } else {
 #pragma unroll
       for (int i = 0; i < n; ++i)
 #pragma unroll
         for (int j = i + 1; j < n; ++j) {
           T f[V];
-          if constexpr (sizeof(T) == 4) {
-            // Rare path (a log ratio of the line outside the series range):
-            // fresh copies of the two records from LDS. The opaque zero offset
-            // keeps them apart from the register copies used by the fast path,
-            // which then die at the branch; reusing them here would set the
-            // register allocation of the whole kernel (144 instead of 106
-            // VGPRs for 3D p3, one wave per SIMD less).
-            int z0 = 0;
-            asm volatile("" : "+v"(z0));
-            const T *sw = s_w + z0;
-            NodeR<T, D> wi, wj;
-            auto read = [&](NodeR<T, D> &x, int q) {
-              x.r = sw[0 * SZ + q];
-              x.lrho = sw[1 * SZ + q];
-              x.b = sw[2 * SZ + q];
-              x.lbeta = sw[3 * SZ + q];
+          // Rare path (a log ratio of the line outside the series range):
+          // fresh copies of the two records from LDS. The opaque zero offset
+          // keeps them apart from the register copies used by the fast path,
+          // which then die at the branch; reusing them here would set the
+          // register allocation of the whole kernel (144 instead of 106
+          // VGPRs for 3D p3, one wave per SIMD less).
+          int z0 = 0;
+          asm volatile("" : "+v"(z0));
+          const T *sw = s_w + z0;
+          NodeR<T, D> wi, wj;
+          auto read = [&](NodeR<T, D> &x, int q) {
+            x.r = sw[0 * SZ + q];
+            x.lrho = sw[1 * SZ + q];
+            x.b = sw[2 * SZ + q];
+            x.lbeta = sw[3 * SZ + q];
 #pragma unroll
-              for (int d = 0; d < D; ++d) x.h[d] = sw[(4 + d) * SZ + q];
-              x.hp = sw[(4 + D) * SZ + q];
-            };
-            read(wi, pq[i]);
-            read(wj, pq[j]);
-            flux_ranocha_r<T, D, O, SQ>(wi, wj, igm1, f);
-          } else {
-            flux_ranocha_r<T, D, O, SQ>(w[i], w[j], igm1, f);
-          }
+            for (int d = 0; d < D; ++d) x.h[d] = sw[(4 + d) * SZ + q];
+            x.hp = sw[(4 + D) * SZ + q];
+          };
+          read(wi, pq[i]);
+          read(wj, pq[j]);
+          flux_ranocha_r<T, D, O, SQ>(wi, wj, igm1, f);
           const T di = k.Dsplit[i * n + j], dj = k.Dsplit[j * n + i];
 #pragma unroll
           for (int v = 0; v < V; ++v) {
@@ -546,10 +665,36 @@ __device__ __forceinline__ void line_work(const ElemArgs<T> &a, const DGConst<T,
         fprev[v] = T(0);
         cur[v] = s_c[v * SZ + pq[0]];
       }
+      // FP64 shock capturing with LLF subcell fluxes: primitive variables and
+      // sound speeds from the node records (no division and no square root)
+      constexpr bool FROM_W = F64 && VT::HG && VT::RAN;
+      const bool llf = FROM_W && (a.fv_flux == FLUX_LLF || a.fv_flux == FLUX_LLF_NAIVE);
+      ConsP<T, D> pcur;
+      T ccur = T(0);
+      if constexpr (FROM_W) {
+        if (llf) {
+          NodeD<D> w0;
+          load_record<D, SZ>(w0, s_w, pq[0]);
+          consp_from_node<D>(cur, w0, a.sqrt_gamma, pcur, ccur);
+        }
+      }
 #pragma unroll
       for (int i = 0; i < n; ++i) {
         T fnext[V];
-        if (i < n - 1) {
+        if (FROM_W && llf && i < n - 1) {
+          if constexpr (FROM_W) {
+            NodeD<D> w1;
+            ConsP<T, D> pnxt;
+            T nxt[V], cnxt;
+#pragma unroll
+            for (int v = 0; v < V; ++v) nxt[v] = s_c[v * SZ + pq[i + 1]];
+            load_record<D, SZ>(w1, s_w, pq[i + 1]);
+            consp_from_node<D>(nxt, w1, a.sqrt_gamma, pnxt, cnxt);
+            flux_llf_pc<T, D, O>(pcur, pnxt, ccur, cnxt, a.fv_flux == FLUX_LLF_NAIVE, fnext);
+            pcur = pnxt;
+            ccur = cnxt;
+          }
+        } else if (i < n - 1) {
           T nxt[V];
 #pragma unroll
           for (int v = 0; v < V; ++v) nxt[v] = s_c[v * SZ + pq[i + 1]];
@@ -570,15 +715,6 @@ __device__ __forceinline__ void line_work(const ElemArgs<T> &a, const DGConst<T,
     }
   }
 
-  // keep the face work (which waits on the neighbour loads of phase A) behind
-  // the volume arithmetic
-  __builtin_amdgcn_sched_barrier(0);
-  faces();
-
-#pragma unroll
-  for (int i = 0; i < n; ++i)
-#pragma unroll
-    for (int v = 0; v < V; ++v) s_d[(O * V + v) * SZ + pq[i]] = acc[i][v];
 }
 
 // Source-term phase tables of one element: with x_d = c_d + J xi_{i_d} the
@@ -614,33 +750,49 @@ __device__ __forceinline__ void source_table_entry(const DGConst<T, N> &k, int i
   tab[2 * idx + 1] = co;
 }
 
-// LDS region A of a variant (node records and/or conservative state, later the
-// output staging), in elements of T
-template <typename T, int D, int N, int VOL, int EPB> constexpr int region_a_size() {
-  constexpr int NW = VolTraits<VOL>::RAN ? nodeR_count(D) : 0;
-  constexpr int NC = VolTraits<VOL>::CONS ? D + 2 : 0;
-  constexpr int ALIGN = 16 / (int)sizeof(T);
-  return ((NW + NC) * Layout<D, N, EPB>::SIZE + ALIGN - 1) / ALIGN * ALIGN;
-}
-// The fused last stage can reduce the wave speed when region A holds the D
-// per-node FP64 speeds of the tile (not so for the weak form, central flux and
-// pure FV in 3D FP32, whose region A is the conservative state only).
-template <typename T, int D, int N, int VOL, int EPB> constexpr bool stage_speed_fits() {
-  return (size_t)region_a_size<T, D, N, VOL, EPB>() * sizeof(T) >=
-         (size_t)D * EPB * ipow_c(N + 1, D) * sizeof(double);
-}
-// The fused stage of a 2D polydeg-3 shock-capturing variant can compute the
-// next stage's indicator when the tile is whole wavefronts of 16 elements, one
-// wavefront each, and region A holds their 512 doubles of scratch apiece.
-template <typename T, int D, int N, int VOL, int EPB, int NT> constexpr bool stage_ind2d_fits() {
-  return D == 2 && N == 3 && VolTraits<VOL>::HG && EPB % 16 == 0 && EPB / 16 <= NT / 64 &&
-         (size_t)region_a_size<T, D, N, VOL, EPB>() * sizeof(T) >= (size_t)(EPB / 16) * 512 * sizeof(double);
-}
+// LDS of a variant, in bytes. Phases A and B hold the staged tile [q][v] and the
+// node records (records of flux_ranocha and/or the conservative state by
+// variable); the line results of the D directions take the tile's memory after
+// phase B. In FP64 in 3D they take the records' memory too, the output tile
+// theirs after phase C, and a fused stage's epilogue has its scratch (node wave
+// speeds or indicator sums) at offset 0 and the new state behind it: 3D polydeg
+// 3 falls from 48 to 34 KB, three to four workgroups per CU, which the registers
+// allow. Elsewhere the records keep their own memory, where the output tile goes
+// without the barrier and the registers that the shared one costs (FP32 3D p3
+// RHS 26.2 against 25.1 us; 2D meshes do not fill the chip).
+template <typename T, int D, int N, int VOL, int EPB, int WPD, bool STAGE> struct ElemLds {
+  static constexpr size_t align16(size_t x) { return (x + 15) / 16 * 16; }
+  static constexpr size_t max2(size_t x, size_t y) { return x > y ? x : y; }
+  static constexpr int NQ = EPB * ipow_c(N + 1, D), V = D + 2, SZ = Layout<D, N, EPB>::SIZE;
+  static constexpr int NW = VolTraits<VOL>::RAN ? node_record_size<T, D>() : 0;
+  static constexpr int NC = VolTraits<VOL>::CONS ? V : 0;
+  static constexpr size_t TILE = align16((size_t)NQ * V * sizeof(T));
+  static constexpr size_t RECORDS = align16((size_t)(NW + NC) * SZ * sizeof(T));
+  static constexpr size_t LINES = (size_t)D * V * SZ * sizeof(T);
+  // The fused stage of a 2D polydeg-3 shock-capturing variant can compute the
+  // next stage's indicator when the tile is whole wavefronts of 16 elements,
+  // one wavefront each (512 doubles of scratch apiece).
+  static constexpr bool IND2D =
+      STAGE && D == 2 && N == 3 && VolTraits<VOL>::HG && EPB % 16 == 0 && EPB / 16 <= D * WPD;
+  static constexpr size_t SCRATCH =
+      max2((size_t)D * NQ * sizeof(double), IND2D ? (size_t)(EPB / 16) * 512 * sizeof(double) : 0);
+  static constexpr size_t NEW = STAGE ? align16((size_t)NQ * V * sizeof(double)) : 0;  // new state of a fused stage
+  static constexpr bool SHARE = sizeof(T) == 8 && D == 3;
+  // logarithms behind the records, or between the tile and them
+  static constexpr size_t LOGS =
+      VolTraits<VOL>::RAN && sizeof(T) == 8 ? (size_t)2 * (N + 1) * D * WPD * 64 * sizeof(T) : 0;
+  static constexpr size_t OFF_RECORDS = SHARE ? TILE : align16(max2(max2(TILE + LOGS, LINES), NEW));
+  static constexpr size_t OFF_LOGS = SHARE ? TILE + RECORDS : TILE;
+  static constexpr size_t OFF_OUT = SHARE ? 0 : OFF_RECORDS;  // output tile, later the epilogue's scratch
+  static constexpr size_t OFF_NEW = SHARE ? align16(max2(TILE, SCRATCH)) : 0;
+  static constexpr size_t BYTES =
+      SHARE ? align16(max2(max2(TILE + RECORDS + LOGS, LINES), STAGE ? OFF_NEW + NEW : 0))
+            : OFF_RECORDS + max2(max2(RECORDS, TILE), STAGE ? SCRATCH : 0);
+};
 
 // Wave-speed reduction of the fused last stage (max_speed_nodes_kernel,
 // dg_aux.hpp, for the tile's new state): per node the FP64 wave speeds of
-// node_wave_speeds into s_lam [D][EPB NN] (LDS region A, free after the
-// update), per (element, direction) the maximum over the nodes (S threads per
+// node_wave_speeds into s_lam [D][EPB NN], per (element, direction) the maximum over the nodes (S threads per
 // pair, then one), per element inv_jac * sum over d, and the NaN-propagating
 // maximum over the tile to speed_partial[e0 / EPB]. Maxima are exact, so the
 // partials combine to the same maximum as the stand-alone kernel's.
@@ -652,7 +804,7 @@ __device__ __forceinline__ void stage_wave_speed(const ElemArgs<T> &a, const dou
   __shared__ double s_pm[NPAIR * S];
   __shared__ double s_em[EPB];
   const int tid = threadIdx.x;
-  __syncthreads();  // s_un complete; region A (s_o) no longer read
+  __syncthreads();  // s_un complete; s_lam (shared with the output tile) no longer read
   for (int q = tid; q < ne * NN; q += NT) {
     double lam[D];
     node_wave_speeds<D>([&](int v) { return s_un[q * V + v]; }, a.gamma64, lam);
@@ -691,12 +843,12 @@ __device__ __forceinline__ void stage_wave_speed(const ElemArgs<T> &a, const dou
 // The next stage's indicator of a 2D polydeg-3 tile, from its new state in
 // LDS (s_un, FP64 [q][v]; in FP32 mode rounded to the FP32 state the next
 // stage reads): one wavefront per 16 elements runs indicator_2d_p3_wave with
-// the network operands read where used, s_tmp (region A) holding its 512
+// the network operands read where used, s_tmp holding its 512
 // doubles of scratch per wavefront.
 template <typename T, int EPB>
 __device__ __forceinline__ void stage_indicator_2d(const ElemArgs<T> &a, const double *s_un, double *s_tmp, int ne,
                                                    int e0) {
-  __syncthreads();  // s_un complete; region A no longer read
+  __syncthreads();  // s_un complete; s_tmp no longer read
   const int w = threadIdx.x >> 6;
   if (w < EPB / 16 && w * 16 < ne) {
     const int l = threadIdx.x & 63, el = l & 15, j = l >> 4;
@@ -714,12 +866,11 @@ __device__ __forceinline__ void stage_indicator_2d(const ElemArgs<T> &a, const d
 // issued before the first one is consumed: neighbour ids, the tile (in chunks,
 // into registers), the per-element scalars, then the neighbour face states,
 // which stay in flight until phase B.
-// Minimum wavefronts per SIMD the register allocation must allow. The FP64 3D
-// polydeg-3 flux_ranocha variants are held to 168 VGPRs (from 184, some values
-// spilled): 3 instead of 2 waves per SIMD, RHS 108.9 -> 102.4 us and CK2N54
-// step 613.5 -> 574.7 us on C2 (A/B on one box); no constraint elsewhere.
+// Minimum wavefronts per SIMD the register allocation must allow: the FP64 3D
+// flux_ranocha variants are held to 168 VGPRs, which their means without
+// logarithms meet; the rarely run ones with logarithms spill a few values.
 template <typename T, int D, int N, int VOL> constexpr int min_waves_per_simd() {
-  return sizeof(T) == 8 && D == 3 && N == 3 && VOL == VOL_FD_RANOCHA ? 3 : 1;
+  return sizeof(T) == 8 && D == 3 && VOL == VOL_FD_RANOCHA ? 3 : 1;
 }
 
 template <typename T, int D, int N, int VOL, int EPB, int WPD, bool BND, bool STAGE>
@@ -731,25 +882,20 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
   using C = typename TIO::C;
   constexpr int NT = D * WPD * 64;
   constexpr int n = N + 1, NN = LY::NN, V = D + 2, SZ = LY::SIZE;
-  constexpr int NW = VT::RAN ? nodeR_count(D) : 0;
-  constexpr int NC = VT::CONS ? V : 0;
-  constexpr int ALIGN = 16 / (int)sizeof(T);
-  // primitive / conservative data, later output staging; a multiple of 16 bytes
-  constexpr int SIZE_A = region_a_size<T, D, N, VOL, EPB>();
-  static_assert(SIZE_A == ((NW + NC) * SZ + ALIGN - 1) / ALIGN * ALIGN, "region A");
-  constexpr int SIZE_B = D * V * SZ;  // du per direction, earlier input staging
-  static_assert(SIZE_A >= EPB * NN * V && SIZE_B >= EPB * NN * V, "staging does not fit");
+  using LDS = ElemLds<T, D, N, VOL, EPB, WPD, STAGE>;
   static_assert(EPB * LY::L <= WPD * 64, "one line per lane");
   static_assert(EPB * 2 * n <= NT, "one source-table entry per thread");
   constexpr int RPT = (TIO::NCH + NT - 1) / NT;  // tile chunks per thread
-  __shared__ __attribute__((aligned(16))) T smem[SIZE_A + SIZE_B];
+  __shared__ __attribute__((aligned(16))) unsigned char smem[LDS::BYTES];
   __shared__ double s_alpha[VT::HG ? EPB : 1];
   __shared__ T s_src[EPB * 4 * n];  // per element: (sin, cos) of alpha_i, gamma_j
   __shared__ T s_fac[EPB];          // per element: -inverse_jacobian
-  T *s_w = smem;            // [NW][SZ]
-  T *s_c = smem + NW * SZ;  // [NC][SZ]
-  T *s_d = smem + SIZE_A;   // [D][V][SZ]
-  T *s_o = smem;            // [EPB*NN][V] output staging (region A, free after phase B)
+  T *s_t = reinterpret_cast<T *>(smem);                     // staged tile [EPB*NN][V]
+  T *s_w = reinterpret_cast<T *>(smem + LDS::OFF_RECORDS);  // [NW][SZ]
+  T *s_c = s_w + LDS::NW * SZ;                              // [NC][SZ]
+  T *s_l = reinterpret_cast<T *>(smem + LDS::OFF_LOGS);     // [2 n][NT] logarithms (FP64 flux_ranocha)
+  T *s_d = reinterpret_cast<T *>(smem);                     // [D][V][SZ] line results, after phase B
+  T *s_o = reinterpret_cast<T *>(smem + LDS::OFF_OUT);      // [EPB*NN][V] output, after phase C
 
   const int tid = threadIdx.x;
   // direction of this wave group (wave-uniform, kept in a scalar register)
@@ -778,9 +924,11 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
     for (int r = 0; r < RPT; ++r) {
       const int ic = min(tid + r * NT, nch - 1);
       T x[WC];
+      C cx;
 #pragma unroll
       for (int w = 0; w < WC; ++w) x[w] = T(src64[(size_t)ic * WC + w]);
-      __builtin_memcpy(&rc[r], x, sizeof(C));
+      __builtin_memcpy(&cx, x, sizeof(C));
+      rc[r] = cx;
     }
   } else {
 #pragma unroll
@@ -801,14 +949,14 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
   {
     // lanes past the last chunk rewrite that chunk with the value it holds
     // (an unconditional store keeps the loads above where they are issued)
-    C *dst = reinterpret_cast<C *>(s_d);
+    C *dst = reinterpret_cast<C *>(s_t);
 #pragma unroll
     for (int r = 0; r < RPT; ++r) dst[min(tid + r * NT, nch - 1)] = rc[r];
     if (!full) {  // the bytes of a partial tile past its last whole chunk
       const T *src = a.u + (size_t)e0 * NN * V;
       const double *src64 = u64 ? u64 + (size_t)e0 * NN * V : nullptr;
       for (int i = nch * (TIO::CB / (int)sizeof(T)) + tid; i < ne * NN * V; i += NT)
-        s_d[i] = src64 ? T(src64[i]) : src[i];
+        s_t[i] = src64 ? T(src64[i]) : src[i];
     }
   }
   if constexpr (VT::HG) {
@@ -842,21 +990,27 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
     }
   }
   __syncthreads();
-  if (grp == 0) line_own<T, D, N, EPB, 0>(s_d, lc);
-  else if (grp == 1) line_own<T, D, N, EPB, 1>(s_d, lc);
-  else if constexpr (D == 3) line_own<T, D, N, EPB, 2>(s_d, lc);
   {
     const T gm1 = a.gamma - T(1);
     for (int q = tid; q < ne * NN; q += NT) {
       const int p = LY::phys(q);
       T uq[V];
 #pragma unroll
-      for (int v = 0; v < V; ++v) uq[v] = s_d[q * V + v];
+      for (int v = 0; v < V; ++v) uq[v] = s_t[q * V + v];
       if constexpr (VT::CONS) {
 #pragma unroll
         for (int v = 0; v < V; ++v) s_c[v * SZ + p] = uq[v];
       }
-      if constexpr (VT::RAN) {
+      if constexpr (VT::RAN && sizeof(T) == 8) {
+        NodeD<D> w;
+        nodeD_from_cons<D>(uq, gm1, w);
+        s_w[0 * SZ + p] = w.r;
+        s_w[1 * SZ + p] = w.t;
+#pragma unroll
+        for (int d = 0; d < D; ++d) s_w[(2 + d) * SZ + p] = w.h[d];
+        s_w[(2 + D) * SZ + p] = w.hp;
+      }
+      if constexpr (VT::RAN && sizeof(T) == 4) {
         NodeR<T, D> w;
         nodeR_from_cons<T, D, node_sqrt_rep<T, N>()>(uq, gm1, w);
         s_w[0 * SZ + p] = w.r;
@@ -872,9 +1026,38 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
   __syncthreads();
 
   // ---- phase B: one direction per wave group, one line per lane ----
-  if (grp == 0) line_work<T, D, N, VOL, EPB, 0, BND>(a, k, lc, s_w, s_c, s_d, s_alpha);
-  else if (grp == 1) line_work<T, D, N, VOL, EPB, 1, BND>(a, k, lc, s_w, s_c, s_d, s_alpha);
-  else if constexpr (D == 3) line_work<T, D, N, VOL, EPB, 2, BND>(a, k, lc, s_w, s_c, s_d, s_alpha);
+  T acc[n][V];
+#pragma unroll
+  for (int i = 0; i < n; ++i)
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[i][v] = T(0);
+  LineRecord<T, D, N> wend[2];
+  int pq[n];
+  // calls f with the wave group's direction as a compile-time constant
+  auto in_direction = [&](auto &&f) {
+    if (grp == 0) f(std::integral_constant<int, 0>{});
+    else if (grp == 1) f(std::integral_constant<int, 1>{});
+    else if constexpr (D == 3) f(std::integral_constant<int, 2>{});
+  };
+  if (lc.valid) {
+    in_direction([&](auto o) {
+      line_volume<T, D, N, VOL, EPB, NT, o.value>(a, k, lc, s_w, s_c, s_alpha, s_l + tid, wend, pq, acc);
+      // keep the face work (which waits on the neighbour loads of phase A)
+      // behind the volume arithmetic
+      __builtin_amdgcn_sched_barrier(0);
+      line_faces<T, D, N, VOL, EPB, o.value, BND>(a, k, lc, s_t, s_w, wend, acc);
+    });
+  }
+  __syncthreads();  // the line results take the memory of the tile (FP64: and of the records)
+  if (lc.valid) {
+    if constexpr (LDS::SHARE)  // computed again: held over phase B they cost registers
+      in_direction([&](auto o) { line_slots<D, N, EPB, o.value>(lc.el * NN + lc.base, pq); });
+    T *dst = s_d + grp * V * SZ;
+#pragma unroll
+    for (int i = 0; i < n; ++i)
+#pragma unroll
+      for (int v = 0; v < V; ++v) dst[v * SZ + pq[i]] = acc[i][v];
+  }
   __syncthreads();
 
   // ---- phase C: sum directions, Jacobian, sources; stage the output ----
@@ -898,11 +1081,16 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
       }
     }
   }
-  for (int q = tid; q < ne * NN; q += NT) {
+  constexpr int QPT = (EPB * NN + NT - 1) / NT;  // nodes per thread
+  T dsum[LDS::SHARE ? QPT : 1][V];
+#pragma unroll
+  for (int r = 0; r < QPT; ++r) {
+    const int q = tid + r * NT;
+    if (q >= ne * NN) continue;
     const int el = q / NN, node = q - el * NN;
     const int p = LY::phys(q);
     const T fac = s_fac[el];
-    T d[V];
+    T *d = dsum[LDS::SHARE ? r : 0];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
       T sum = s_d[(0 * V + v) * SZ + p];
@@ -932,22 +1120,32 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
 #pragma unroll
       for (int v = 0; v < V; ++v) d[v] += s[v];
     }
+    if constexpr (!LDS::SHARE) {
 #pragma unroll
-    for (int v = 0; v < V; ++v) s_o[q * V + v] = d[v];
+      for (int v = 0; v < V; ++v) s_o[q * V + v] = d[v];
+    }
   }
   __syncthreads();
+  if constexpr (LDS::SHARE) {  // the line results are read: their memory takes the output tile
+#pragma unroll
+    for (int r = 0; r < QPT; ++r) {
+      const int q = tid + r * NT;
+      if (q >= ne * NN) continue;
+#pragma unroll
+      for (int v = 0; v < V; ++v) s_o[q * V + v] = dsum[r][v];
+    }
+    __syncthreads();
+  }
   if constexpr (STAGE) {
     // the 2N update of the tile's values, in the same arithmetic as
     // rk2n_update_kernel (bitwise equal to the unfused stage); with the speed
-    // reduction the new values are kept in LDS too (region B, [q][v], free
-    // after phase C)
+    // reduction or the indicator the new values are kept in LDS too ([q][v])
     const double b_dt = a.tdev ? a.b_stage * a.tdev[1] : a.b_stage;
-    constexpr bool SPEED_FITS = stage_speed_fits<T, D, N, VOL, EPB>();
-    const bool speed = SPEED_FITS && a.speed_partial != nullptr;
-    constexpr bool IND2D = stage_ind2d_fits<T, D, N, VOL, EPB, NT>();
+    const bool speed = a.speed_partial != nullptr;
+    constexpr bool IND2D = LDS::IND2D;
     const bool ind = IND2D && a.ind_next != 0;
-    double *s_un = reinterpret_cast<double *>(s_d);
-    static_assert(SIZE_B * sizeof(T) >= (size_t)EPB * NN * V * sizeof(double), "new state staging does not fit");
+    double *s_un = reinterpret_cast<double *>(smem + LDS::OFF_NEW);
+    double *s_tmp = reinterpret_cast<double *>(smem + LDS::OFF_OUT);
     auto update = [&](size_t g, T du_v, double ut, double ur) {
       ut = double(du_v) - ut * a.a_stage;
       const double un = tfma(ut, b_dt, ur);
@@ -972,11 +1170,9 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
         update(g, s_o[i], a.first_stage ? 0.0 : double(a.u_tmp[g]), a.u_reg_in[g]);
       }
     }
-    if constexpr (SPEED_FITS) {
-      if (speed) stage_wave_speed<T, D, N, EPB, NT>(a, s_un, reinterpret_cast<double *>(smem), ne, e0);
-    }
+    if (speed) stage_wave_speed<T, D, N, EPB, NT>(a, s_un, s_tmp, ne, e0);
     if constexpr (IND2D) {
-      if (ind) stage_indicator_2d<T, EPB>(a, s_un, reinterpret_cast<double *>(smem), ne, e0);
+      if (ind) stage_indicator_2d<T, EPB>(a, s_un, s_tmp, ne, e0);
     }
   } else if (full) {
     const C *src = reinterpret_cast<const C *>(s_o);

@@ -29,8 +29,8 @@ struct ElemKey {
 using ElemLaunch = hipError_t (*)(const void *args, const void *kconst, int nblocks, hipStream_t s);
 
 std::map<ElemKey, ElemLaunch> &elem_registry();  // defined in trixi_hip.hip
-// what a fused-stage variant's epilogue can add: the wave-speed reduction
-// (stage_speed_fits) and the next stage's 2D p3 indicator (stage_ind2d_fits)
+// what a fused-stage variant's epilogue can add: the wave-speed reduction and
+// the next stage's 2D p3 indicator
 struct ElemCaps {
   bool speed = false, ind2d = false;
 };
@@ -49,8 +49,7 @@ template <typename T, int D, int N, int VOL, int EPB, int WPD, bool BND, bool ST
   Reg() {
     const ElemKey key{sizeof(T) == 4, D, N, VOL, EPB, D * WPD * 64, BND ? 1 : 0, STAGE ? 1 : 0};
     elem_registry()[key] = &launch_elem<T, D, N, VOL, EPB, WPD, BND, STAGE>;
-    elem_caps()[key] = ElemCaps{STAGE && stage_speed_fits<T, D, N, VOL, EPB>(),
-                                STAGE && stage_ind2d_fits<T, D, N, VOL, EPB, D * WPD * 64>()};
+    elem_caps()[key] = ElemCaps{STAGE, ElemLds<T, D, N, VOL, EPB, WPD, STAGE>::IND2D};
   }
 };
 
