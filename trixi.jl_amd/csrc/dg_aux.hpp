@@ -22,8 +22,10 @@ template <int N> struct VinvConst {
   double Vinv[(N + 1) * (N + 1)];
 };
 
-template <typename T, int D, int N, int IPB, int NT>
-__global__ __launch_bounds__(NT) void hg_indicator_kernel(const T *__restrict__ u,
+// T: precision of the state the factors belong to; S: type of the array, rounded
+// to T on load (an FP32 RHS between FP64 arrays).
+template <typename T, int D, int N, int IPB, int NT, typename S>
+__global__ __launch_bounds__(NT) void hg_indicator_kernel(const S *__restrict__ u,
                                                           double *__restrict__ alpha_raw, int E,
                                                           HGParams hp, VinvConst<N> vc) {
   constexpr int n = N + 1, NN = ipow_c(n, D), V = D + 2;
@@ -33,7 +35,9 @@ __global__ __launch_bounds__(NT) void hg_indicator_kernel(const T *__restrict__ 
   if (e0 >= E) return;
   const int ne = min(IPB, E - e0);
   for (int q = tid; q < ne * NN; q += NT) {
-    const T *un = u + (size_t)(e0 * NN + q) * V;
+    T un[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) un[v] = T(u[(size_t)(e0 * NN + q) * V + v]);
     double rho = un[0], m2 = 0;
 #pragma unroll
     for (int d = 0; d < D; ++d) m2 += double(un[1 + d]) * double(un[1 + d]);
@@ -630,8 +634,9 @@ __global__ __launch_bounds__(256) void initial_state_kernel(const double *__rest
 // boundary face node; bnd[b] = {element, 0-based direction}; the flux goes to
 // face slot b of mflux, face node = the element kernel's line index (free
 // indices, lower dimension fastest).
-template <typename T, int D, int N>
-__global__ __launch_bounds__(256) void slip_wall_flux_kernel(const T *__restrict__ u, const int32_t *__restrict__ bnd,
+// The state array is of type S, rounded to T on load.
+template <typename T, int D, int N, typename S>
+__global__ __launch_bounds__(256) void slip_wall_flux_kernel(const S *__restrict__ u, const int32_t *__restrict__ bnd,
                                                              int B, double gamma, T *__restrict__ mflux) {
   constexpr int n = N + 1, V = D + 2, L = D == 3 ? n * n : n, NN = ipow_c(n, D);
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -653,16 +658,21 @@ __global__ __launch_bounds__(256) void slip_wall_flux_kernel(const T *__restrict
     }
   }
   const int node = D == 3 ? idx[0] + n * (idx[1] + n * idx[2]) : idx[0] + n * idx[1];
-  const T *q = u + ((size_t)e * NN + node) * V;
+  T q[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) q[v] = T(u[((size_t)e * NN + node) * V + v]);
   const double rho = double(q[0]);
-  const double mo = double(q[1 + o]);
+  // momenta by constant indices and selects: an indexed register array would
+  // live in scratch memory
+  const double m0 = double(q[1]), m1 = double(q[2]), m2 = D == 3 ? double(q[3]) : 0.0;
+  const double mo = o == 0 ? m0 : o == 1 ? m1 : m2;
   const double mn = plus ? mo : -mo;
   double mt0, mt1 = 0.0;
   if constexpr (D == 3) {
-    mt0 = double(q[1 + (o == 0 ? 2 : (o == 1 ? 0 : 1))]);
-    mt1 = double(q[1 + (o == 0 ? 1 : (o == 1 ? 2 : 0))]);
+    mt0 = o == 0 ? m2 : o == 1 ? m0 : m1;
+    mt1 = o == 0 ? m1 : o == 1 ? m2 : m0;
   } else {
-    mt0 = double(q[1 + (1 - o)]);
+    mt0 = o == 0 ? m1 : m0;
   }
   const double vn = mn / rho;
   double ke2 = mn * vn;
@@ -696,12 +706,13 @@ __global__ __launch_bounds__(256) void slip_wall_flux_kernel(const T *__restrict
 // (S = 2^(D-1) faces of n^(D-1) nodes), MPB mortars per 256-thread block.
 // mort[m] = {small ids [S], large id, orientation, large_side};
 // mflux[(slot * L + node) * V + v], slot = slot0 + m (S + 1) + face (S = large).
+// The state array is of type S_, rounded to T on load.
 template <typename T, int N> struct MortarConst {
   T fu[(N + 1) * (N + 1)], fl[(N + 1) * (N + 1)], ru[(N + 1) * (N + 1)], rl[(N + 1) * (N + 1)];
 };
 
-template <typename T, int D, int N>
-__global__ __launch_bounds__(256) void mortar_flux_kernel(const T *__restrict__ u, const int32_t *__restrict__ mort,
+template <typename T, int D, int N, typename S_>
+__global__ __launch_bounds__(256) void mortar_flux_kernel(const S_ *__restrict__ u, const int32_t *__restrict__ mort,
                                                           int M, int slot0, int surface_flux, T gamma,
                                                           MortarConst<T, N> mc, T *__restrict__ mflux) {
   constexpr int n = N + 1, V = D + 2, S = 1 << (D - 1), L = D == 3 ? n * n : n, NN = ipow_c(n, D);
@@ -726,9 +737,9 @@ __global__ __launch_bounds__(256) void mortar_flux_kernel(const T *__restrict__ 
     return node;
   };
   if (active && r < L) {
-    const T *src = u + ((size_t)large * NN + node_of(r, large_left ? n - 1 : 0)) * V;
+    const S_ *src = u + ((size_t)large * NN + node_of(r, large_left ? n - 1 : 0)) * V;
 #pragma unroll
-    for (int v = 0; v < V; ++v) s_ul[mm][r][v] = src[v];
+    for (int v = 0; v < V; ++v) s_ul[mm][r][v] = T(src[v]);
   }
   __syncthreads();
   if (active) {
@@ -752,10 +763,10 @@ __global__ __launch_bounds__(256) void mortar_flux_kernel(const T *__restrict__ 
         up[v] = acc;
       }
     }
-    const T *us = u + ((size_t)md[q] * NN + node_of(fn, large_left ? 0 : n - 1)) * V;
+    const S_ *us = u + ((size_t)md[q] * NN + node_of(fn, large_left ? 0 : n - 1)) * V;
     T usv[V], f[V];
 #pragma unroll
-    for (int v = 0; v < V; ++v) usv[v] = us[v];
+    for (int v = 0; v < V; ++v) usv[v] = T(us[v]);
     const T *ul = large_left ? up : usv;
     const T *ur = large_left ? usv : up;
     if (o == 0) num_flux_c<T, D, 0, true>(surface_flux, ul, ur, gamma, f);

@@ -49,6 +49,12 @@ template <typename T, int N> struct DGConst {
   double nodes[n];  // LGL nodes (coordinates of sources)
 };
 
+// What an element kernel does with the result: store du, apply the 2N stage
+// update, or (FP32) the RHS between FP64 arrays. The last is a variant of its
+// own: as run-time branches of the first it cost the native RHS 6 % (24.8 against
+// 26.3 us, 3D p3 on 32^3 elements).
+enum ElemMode { ELEM_RHS = 0, ELEM_STAGE = 1, ELEM_RHS64 = 2 };
+
 template <typename T> struct ElemArgs {
   const T *__restrict__ u;               // [V, NN, E]
   T *__restrict__ du;                    // [V, NN, E]
@@ -88,6 +94,12 @@ template <typename T> struct ElemArgs {
   double *u_reg_out;
   float *u32_out;
   const double *u64;
+  // FP32 RHS between FP64 arrays (RHS64 variants): u64 as above, also with
+  // mortars and slip walls, whose fluxes are given (null: the state is u), and
+  // the results widened into du64. Without a rounded copy of the state and an
+  // FP32 result a call moves 16 bytes per value instead of 40 (3D p3 on 32^3
+  // elements: 73.9 us in three launches, 52.0 us in one).
+  double *du64;
   double a_stage, b_stage;
   int first_stage;
   T gamma;
@@ -133,6 +145,53 @@ template <typename T, int D, int N, int EPB> struct TileIO {
   using C = typename ChunkOf<CB>::type;
   static constexpr int NCH = TB / CB;
 };
+
+// W consecutive values between global memory (aligned to the smaller of 16 and
+// W sizeof(S) bytes) and registers, in pieces of up to 16 bytes. A fused stage
+// that moved its registers value by value, 4 and 8 bytes at strides of 16 and 32,
+// was bound by the number of its memory accesses: FP32 3D p3 stage 70.4 -> 54 us,
+// FP64 98 -> 90 us (32^3 elements; 252 and 420 MB).
+template <typename S, int W> struct Pieces {
+  static constexpr int K = 16 / (int)sizeof(S) < W ? 16 / (int)sizeof(S) : W;
+  typedef S V __attribute__((ext_vector_type(K > 1 ? K : 2)));
+};
+template <int W, typename S> __device__ __forceinline__ void load_values(const S *p, S (&x)[W]) {
+  using P = Pieces<S, W>;
+  if constexpr (P::K == 1) {
+#pragma unroll
+    for (int w = 0; w < W; ++w) x[w] = p[w];
+  } else {
+    using Vec = typename P::V;
+#pragma unroll
+    for (int w = 0; w < W; w += P::K) {
+      const Vec v = *reinterpret_cast<const Vec *>(p + w);
+#pragma unroll
+      for (int j = 0; j < P::K; ++j) x[w + j] = v[j];
+    }
+  }
+}
+template <int W, typename S> __device__ __forceinline__ void store_values(S *p, const S (&x)[W]) {
+  using P = Pieces<S, W>;
+  if constexpr (P::K == 1) {
+#pragma unroll
+    for (int w = 0; w < W; ++w) p[w] = x[w];
+  } else {
+    using Vec = typename P::V;
+#pragma unroll
+    for (int w = 0; w < W; w += P::K) {
+      Vec v;
+#pragma unroll
+      for (int j = 0; j < P::K; ++j) v[j] = x[w + j];
+      *reinterpret_cast<Vec *>(p + w) = v;
+    }
+  }
+}
+// x, available here: keeps the compiler from moving what is computed from a
+// loaded value up to its load, in front of the loads issued after it
+__device__ __forceinline__ double here(double x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
 
 // LDS index map and lane -> line assignment (see the header comment).
 template <int D, int N, int EPB> struct Layout {
@@ -231,18 +290,17 @@ __device__ __forceinline__ void line_loads(const ElemArgs<T> &a, LineCtx<T, D + 
   constexpr int n = N + 1, NN = LY::NN, V = D + 2, L = LY::L;
   const int st = o == 0 ? 1 : (o == 1 ? n : n * n);
   if constexpr (sizeof(T) == 4) {
-    if (u64) {  // FP32 stage reading the FP64 register (wave-uniform)
-      // With BND only boundary faces (no mortar or slip-wall slots) occur
-      // here: their outer state is the ghost record, loaded in FP32 beside the
-      // (clamped, in-bounds) register load and selected per lane.
+    if (u64) {  // FP32 stage or RHS reading an FP64 state (wave-uniform)
+      // With BND the outer state at a face slot is the ghost record, loaded in
+      // FP32 beside the (clamped, in-bounds) FP64 load and selected per lane.
       const bool im = !BND || nbm >= 0, ip = !BND || nbp >= 0;
       const double *vm = u64 + ((size_t)(im ? nbm : 0) * NN + c.base + (n - 1) * st) * V;
       const double *vp = u64 + ((size_t)(ip ? nbp : 0) * NN + c.base) * V;
       if constexpr (BND) {
         const T *gm = a.ghost + ((size_t)(im ? 0 : -nbm - 1) * L + c.line) * V;
         const T *gp = a.ghost + ((size_t)(ip ? 0 : -nbp - 1) * L + c.line) * V;
-        c.fm = -1;
-        c.fp = -1;
+        c.fm = (!im && -nbm - 1 >= a.nbnd) ? ((-nbm - 1) * L + c.line) * V : -1;
+        c.fp = (!ip && -nbp - 1 >= a.nbnd) ? ((-nbp - 1) * L + c.line) * V : -1;
 #pragma unroll
         for (int v = 0; v < V; ++v) {
           const T xm = T(vm[v]), gmv = gm[v], xp = T(vp[v]), gpv = gp[v];
@@ -760,7 +818,8 @@ __device__ __forceinline__ void source_table_entry(const DGConst<T, N> &k, int i
 // allow. Elsewhere the records keep their own memory, where the output tile goes
 // without the barrier and the registers that the shared one costs (FP32 3D p3
 // RHS 26.2 against 25.1 us; 2D meshes do not fill the chip).
-template <typename T, int D, int N, int VOL, int EPB, int WPD, bool STAGE> struct ElemLds {
+template <typename T, int D, int N, int VOL, int EPB, int WPD, int MODE> struct ElemLds {
+  static constexpr bool STAGE = MODE == ELEM_STAGE;
   static constexpr size_t align16(size_t x) { return (x + 15) / 16 * 16; }
   static constexpr size_t max2(size_t x, size_t y) { return x > y ? x : y; }
   static constexpr int NQ = EPB * ipow_c(N + 1, D), V = D + 2, SZ = Layout<D, N, EPB>::SIZE;
@@ -873,7 +932,7 @@ template <typename T, int D, int N, int VOL> constexpr int min_waves_per_simd() 
   return sizeof(T) == 8 && D == 3 && VOL == VOL_FD_RANOCHA ? 3 : 1;
 }
 
-template <typename T, int D, int N, int VOL, int EPB, int WPD, bool BND, bool STAGE>
+template <typename T, int D, int N, int VOL, int EPB, int WPD, bool BND, int MODE>
 __global__ __launch_bounds__(D *WPD * 64) __attribute__((amdgpu_waves_per_eu(min_waves_per_simd<T, D, N, VOL>())))
 void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
   using LY = Layout<D, N, EPB>;
@@ -882,7 +941,9 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
   using C = typename TIO::C;
   constexpr int NT = D * WPD * 64;
   constexpr int n = N + 1, NN = LY::NN, V = D + 2, SZ = LY::SIZE;
-  using LDS = ElemLds<T, D, N, VOL, EPB, WPD, STAGE>;
+  using LDS = ElemLds<T, D, N, VOL, EPB, WPD, MODE>;
+  constexpr bool STAGE = MODE == ELEM_STAGE, RHS64 = MODE == ELEM_RHS64;
+  static_assert(!RHS64 || sizeof(T) == 4, "the RHS between FP64 arrays is a variant of FP32");
   static_assert(EPB * LY::L <= WPD * 64, "one line per lane");
   static_assert(EPB * 2 * n <= NT, "one source-table entry per thread");
   constexpr int RPT = (TIO::NCH + NT - 1) / NT;  // tile chunks per thread
@@ -914,21 +975,18 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
   // chunk indices are clamped to the tile's extent, so all lanes load (a
   // partial last tile is staged by the scalar loop below instead)
   const int nch = full ? TIO::NCH : max(1, ne * NN * V * (int)sizeof(T) / TIO::CB);
-  const double *u64 = STAGE && sizeof(T) == 4 ? a.u64 : nullptr;  // FP64 source of the FP32 stage, or null
+  const double *u64 = sizeof(T) == 4 && (STAGE || RHS64) ? a.u64 : nullptr;  // FP64 source of an FP32 variant, or null
   const C *csrc = reinterpret_cast<const C *>(a.u + (size_t)e0 * NN * V);
   C rc[RPT];
-  if (STAGE && sizeof(T) == 4 && u64) {
-    constexpr int WC = TIO::CB / (int)sizeof(T);
+  constexpr int WC = TIO::CB / (int)sizeof(T);  // values per chunk
+  constexpr bool CAN64 = sizeof(T) == 4 && (STAGE || RHS64);
+  double r64[CAN64 ? RPT : 1][WC];
+  if (CAN64 && u64) {
     const double *src64 = u64 + (size_t)e0 * NN * V;
 #pragma unroll
     for (int r = 0; r < RPT; ++r) {
       const int ic = min(tid + r * NT, nch - 1);
-      T x[WC];
-      C cx;
-#pragma unroll
-      for (int w = 0; w < WC; ++w) x[w] = T(src64[(size_t)ic * WC + w]);
-      __builtin_memcpy(&cx, x, sizeof(C));
-      rc[r] = cx;
+      load_values<WC>(src64 + (size_t)ic * WC, r64[r]);
     }
   } else {
 #pragma unroll
@@ -950,8 +1008,22 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
     // lanes past the last chunk rewrite that chunk with the value it holds
     // (an unconditional store keeps the loads above where they are issued)
     C *dst = reinterpret_cast<C *>(s_t);
+    if (CAN64 && u64) {
+      // rounded here: with the rounding beside the loads, the neighbour states
+      // were asked for after the wait for the tile
 #pragma unroll
-    for (int r = 0; r < RPT; ++r) dst[min(tid + r * NT, nch - 1)] = rc[r];
+      for (int r = 0; r < RPT; ++r) {
+        T x[WC];
+        C cx;
+#pragma unroll
+        for (int w = 0; w < WC; ++w) x[w] = T(here(r64[r][w]));
+        __builtin_memcpy(&cx, x, sizeof(C));
+        dst[min(tid + r * NT, nch - 1)] = cx;
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < RPT; ++r) dst[min(tid + r * NT, nch - 1)] = rc[r];
+    }
     if (!full) {  // the bytes of a partial tile past its last whole chunk
       const T *src = a.u + (size_t)e0 * NN * V;
       const double *src64 = u64 ? u64 + (size_t)e0 * NN * V : nullptr;
@@ -1063,20 +1135,22 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
   // ---- phase C: sum directions, Jacobian, sources; stage the output ----
   // The fused stage's register loads (u_tmp, u) of a full tile are issued
   // here, all at once, so that their latency overlaps the rest of phase C.
-  constexpr int W = TIO::CB / (int)sizeof(T);  // values per chunk
-  constexpr int NPRE = STAGE ? RPT * W : 1;
-  double pre_t[NPRE], pre_u[NPRE];
+  constexpr int W = WC;
+  constexpr int NPRE = STAGE ? RPT : 1;
+  T pre_t[NPRE][W];
+  double pre_u[NPRE][W];
   const size_t base = (size_t)e0 * NN * V;
   if constexpr (STAGE) {
     if (full) {
 #pragma unroll
       for (int r = 0; r < RPT; ++r) {
         const int ic = min(tid + r * NT, TIO::NCH - 1);  // clamped: every lane loads in bounds
+        load_values<W>(a.u_reg_in + base + (size_t)ic * W, pre_u[r]);
+        if (a.first_stage) {
 #pragma unroll
-        for (int w = 0; w < W; ++w) {
-          const size_t g = base + (size_t)ic * W + w;
-          pre_t[r * W + w] = a.first_stage ? 0.0 : double(a.u_tmp[g]);
-          pre_u[r * W + w] = a.u_reg_in[g];
+          for (int w = 0; w < W; ++w) pre_t[r][w] = T(0);
+        } else {
+          load_values<W>(a.u_tmp + base + (size_t)ic * W, pre_t[r]);
         }
       }
     }
@@ -1146,33 +1220,65 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
     const bool ind = IND2D && a.ind_next != 0;
     double *s_un = reinterpret_cast<double *>(smem + LDS::OFF_NEW);
     double *s_tmp = reinterpret_cast<double *>(smem + LDS::OFF_OUT);
-    auto update = [&](size_t g, T du_v, double ut, double ur) {
-      ut = double(du_v) - ut * a.a_stage;
-      const double un = tfma(ut, b_dt, ur);
-      a.u_tmp[g] = T(ut);
-      a.u_reg_out[g] = un;
-      if (a.u32_out) a.u32_out[g] = float(un);
-      if (speed || ind) s_un[g - base] = un;
+    auto update = [&](T du_v, T ut, double ur, T &ut_new, double &u_new) {
+      const double x = double(du_v) - double(ut) * a.a_stage;
+      u_new = tfma(x, b_dt, ur);
+      ut_new = T(x);
     };
     if (full) {
 #pragma unroll
       for (int r = 0; r < RPT; ++r) {
         const int i = tid + r * NT;
         if (i < TIO::NCH) {
+          T ut[W];
+          double un[W];
 #pragma unroll
-          for (int w = 0; w < W; ++w)
-            update(base + (size_t)i * W + w, s_o[i * W + w], pre_t[r * W + w], pre_u[r * W + w]);
+          for (int w = 0; w < W; ++w) update(s_o[i * W + w], pre_t[r][w], pre_u[r][w], ut[w], un[w]);
+          store_values<W>(a.u_tmp + base + (size_t)i * W, ut);
+          store_values<W>(a.u_reg_out + base + (size_t)i * W, un);
+          if (a.u32_out) {
+            float us[W];
+#pragma unroll
+            for (int w = 0; w < W; ++w) us[w] = float(un[w]);
+            store_values<W>(a.u32_out + base + (size_t)i * W, us);
+          }
+          if (speed || ind) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) s_un[i * W + w] = un[w];
+          }
         }
       }
     } else {
       for (int i = tid; i < ne * NN * V; i += NT) {
         const size_t g = base + i;
-        update(g, s_o[i], a.first_stage ? 0.0 : double(a.u_tmp[g]), a.u_reg_in[g]);
+        T ut;
+        double un;
+        update(s_o[i], a.first_stage ? T(0) : a.u_tmp[g], a.u_reg_in[g], ut, un);
+        a.u_tmp[g] = ut;
+        a.u_reg_out[g] = un;
+        if (a.u32_out) a.u32_out[g] = float(un);
+        if (speed || ind) s_un[i] = un;
       }
     }
     if (speed) stage_wave_speed<T, D, N, EPB, NT>(a, s_un, s_tmp, ne, e0);
     if constexpr (IND2D) {
       if (ind) stage_indicator_2d<T, EPB>(a, s_un, s_tmp, ne, e0);
+    }
+  } else if constexpr (RHS64) {
+    double *dst = a.du64 + base;
+    if (full) {
+#pragma unroll
+      for (int r = 0; r < RPT; ++r) {
+        const int i = tid + r * NT;
+        if (i < TIO::NCH) {
+          double x[W];
+#pragma unroll
+          for (int w = 0; w < W; ++w) x[w] = double(s_o[i * W + w]);
+          store_values<W>(dst + (size_t)i * W, x);
+        }
+      }
+    } else {
+      for (int i = tid; i < ne * NN * V; i += NT) dst[i] = double(s_o[i]);
     }
   } else if (full) {
     const C *src = reinterpret_cast<const C *>(s_o);

@@ -1,4 +1,4 @@
 // F32 element kernels that apply the 2N stage update (default tiles, periodic meshes).
 #include "elem_registry.hpp"
 
-TRIXI_REG_DEFAULTS(float, false, true)
+TRIXI_REG_DEFAULTS(float, false, trixi_hip::ELEM_STAGE)

@@ -257,37 +257,43 @@ __device__ __forceinline__ void indicator_2d_p3_wave(const T *un, int e0, int E,
 // network image, read from global memory once per workgroup instead of once
 // per wavefront (the image is 13 KB; at 128^2 elements that is 3.3 instead of
 // 13 MB of L2 reads per launch).
+// The state array is of type S, rounded to T on load.
 constexpr int kIndWaves = 4;
-template <typename T, bool FEAT>
-__global__ __launch_bounds__(FEAT ? 64 * kIndWaves : 64) void indicator_2d_p3_kernel(const T *__restrict__ u, int E,
+template <typename T, bool FEAT, typename S>
+__global__ __launch_bounds__(FEAT ? 64 * kIndWaves : 64) void indicator_2d_p3_kernel(const S *__restrict__ u, int E,
                                                                                     Ind2DArgs ia) {
-  constexpr int V = 4, W = FEAT ? kIndWaves : 1;
-  __shared__ double s_mx[W][16 * 16];  // x-transformed rows [element][row j][mode i]
-  __shared__ double s_sq[W][16 * 16];  // squared modes [element][a + 4 j]
+  constexpr int V = 4, NWV = FEAT ? kIndWaves : 1;
+  __shared__ double s_mx[NWV][16 * 16];  // x-transformed rows [element][row j][mode i]
+  __shared__ double s_sq[NWV][16 * 16];  // squared modes [element][a + 4 j]
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int el = l & 15, j = l >> 4;
-  const int e0 = (blockIdx.x * W + w) * 16;
+  const int e0 = (blockIdx.x * NWV + w) * 16;
   const int e = e0 + el;
   const int ec = e < E ? e : E - 1;  // lanes past the end compute on the last element, store nothing
   // the lane's four nodes (i + 4 j): 16 contiguous values, loaded at once in
   // 16-byte pieces before the (wave-uniform) choice of the indicator variable
-  constexpr int NCH = 4 * V * (int)sizeof(T) / 16;
-  float4 raw[NCH];
-  const float4 *src = reinterpret_cast<const float4 *>(u + ((size_t)ec * 16 + 4 * j) * V);
+  constexpr int W = 16 / (int)sizeof(S), NCH = 4 * V / W;
+  typedef S Chunk __attribute__((ext_vector_type(W)));
+  const Chunk *src = reinterpret_cast<const Chunk *>(u + ((size_t)ec * 16 + 4 * j) * V);
+  T un[4 * V];
 #pragma unroll
-  for (int c = 0; c < NCH; ++c) raw[c] = src[c];
+  for (int c = 0; c < NCH; ++c) {
+    const Chunk x = src[c];
+#pragma unroll
+    for (int k = 0; k < W; ++k) un[c * W + k] = T(x[k]);
+  }
   if constexpr (FEAT) {
     __shared__ __attribute__((aligned(16))) mlp::InferImage s_img;
     if (ia.net) {  // uniform: copy the image in 16-byte pieces
       constexpr int NC = (int)(sizeof(mlp::InferImage) / 16);
       const float4 *gi = reinterpret_cast<const float4 *>(ia.img);
       float4 *si = reinterpret_cast<float4 *>(&s_img);
-      for (int c = threadIdx.x; c < NC; c += 64 * W) si[c] = gi[c];
+      for (int c = threadIdx.x; c < NC; c += 64 * NWV) si[c] = gi[c];
     }
     __syncthreads();
-    indicator_2d_p3_wave<T, FEAT, true, true>(reinterpret_cast<const T *>(raw), e0, E, ia, s_mx[w], s_sq[w], &s_img);
+    indicator_2d_p3_wave<T, FEAT, true, true>(un, e0, E, ia, s_mx[w], s_sq[w], &s_img);
   } else {
-    indicator_2d_p3_wave<T, FEAT>(reinterpret_cast<const T *>(raw), e0, E, ia, s_mx[w], s_sq[w]);
+    indicator_2d_p3_wave<T, FEAT>(un, e0, E, ia, s_mx[w], s_sq[w]);
   }
 }
 

@@ -143,7 +143,7 @@ struct trixi_hip_ctx {
   void *d_du = nullptr;  // native precision
   // staging for trixi_hip_rhs (FP64 interface)
   double *d_hu = nullptr, *d_hdu = nullptr;
-  float *d_su32 = nullptr, *d_sdu32 = nullptr;
+  float *d_su32 = nullptr;  // FP32 mode: the rounded state of a call whose du and u overlap
   // HG: raw factors (scratch of the RHS and indicator entry points) and the
   // smoothed ones
   double *d_alpha_raw = nullptr, *d_alpha = nullptr;
@@ -479,8 +479,9 @@ Ind2DArgs ind2d_args(const trixi_hip_ctx *ctx, const HGParams &params, bool net,
 // feat != null (2D p3) the learned indicator's features [E][32] too, and with
 // alpha_hg != null the HG factor. 2D p3 runs indicator_2d_p3_kernel, the other
 // (ndims, polydeg) hg_indicator_kernel.
-template <typename T>
-int launch_hg(trixi_hip_ctx *ctx, const T *u, double *alpha_out, float *feat, const HGParams *hp = nullptr,
+// The state array is of type S, rounded to T on load.
+template <typename T, typename S>
+int launch_hg(trixi_hip_ctx *ctx, const S *u, double *alpha_out, float *feat, const HGParams *hp = nullptr,
               bool net = false, double *alpha_hg = nullptr) {
   const HGParams params = hp ? *hp : ctx->hg;
   if (ctx->D == 2 && ctx->N == 3) {
@@ -490,10 +491,10 @@ int launch_hg(trixi_hip_ctx *ctx, const T *u, double *alpha_out, float *feat, co
       // the network buffers exist whenever features or the network are asked
       // for (trixi_hip_mlp_features and trixi_hip_set_indicator allocate them)
       if (!ctx->d_mlp || !ctx->d_mlp_img) return set_err(ctx, TRIXI_HIP_ESTATE, "learned-indicator buffers missing");
-      hipLaunchKernelGGL((indicator_2d_p3_kernel<T, true>), dim3((nb + kIndWaves - 1) / kIndWaves),
+      hipLaunchKernelGGL((indicator_2d_p3_kernel<T, true, S>), dim3((nb + kIndWaves - 1) / kIndWaves),
                          dim3(64 * kIndWaves), 0, ctx->stream, u, ctx->E, ia);
     } else {
-      hipLaunchKernelGGL((indicator_2d_p3_kernel<T, false>), dim3(nb), dim3(64), 0, ctx->stream, u, ctx->E, ia);
+      hipLaunchKernelGGL((indicator_2d_p3_kernel<T, false, S>), dim3(nb), dim3(64), 0, ctx->stream, u, ctx->E, ia);
     }
     HIP_TRY(hipGetLastError());
     return TRIXI_HIP_OK;
@@ -506,7 +507,7 @@ int launch_hg(trixi_hip_ctx *ctx, const T *u, double *alpha_out, float *feat, co
     VinvConst<N> vc{};
     for (int i = 0; i < (N + 1) * (N + 1); ++i) vc.Vinv[i] = ctx->Vinv[i];
     int nb = (ctx->E + IPB - 1) / IPB;
-    hipLaunchKernelGGL((hg_indicator_kernel<T, D, N, IPB, 256>), dim3(nb), dim3(256), 0, ctx->stream, u,
+    hipLaunchKernelGGL((hg_indicator_kernel<T, D, N, IPB, 256, S>), dim3(nb), dim3(256), 0, ctx->stream, u,
                        alpha_out, ctx->E, params, vc);
   });
   if (!ok) return set_err(ctx, TRIXI_HIP_EINVAL, "unsupported (ndims, polydeg) for the indicator");
@@ -524,7 +525,7 @@ int mlp_blocks(int n) {
 // Raw (unsmoothed) blending factors of state u into alpha_out, from the
 // indicator selected by ind_mode.
 // (features, network and fallback in one launch: indicator_2d_p3_kernel).
-template <typename T> int launch_indicator_raw(trixi_hip_ctx *ctx, const T *u, double *alpha_out) {
+template <typename T, typename S> int launch_indicator_raw(trixi_hip_ctx *ctx, const S *u, double *alpha_out) {
   return launch_hg<T>(ctx, u, alpha_out, nullptr, nullptr, ctx->ind_mode != TRIXI_HIP_IND_HG);
 }
 
@@ -544,16 +545,17 @@ bool stage_reads_u64(const trixi_hip_ctx *c) {
   return c->fp32 && c->M == 0 && !c->slip && (!is_hg(c) || stage_fuses_indicator(c));
 }
 
-template <typename T>
-int launch_rhs_T(trixi_hip_ctx *ctx, T *du, const T *u, double t, const double *tdev,
-                 const StageOut *so = nullptr) {
+// What the element kernel reads besides the state u (array type S, rounded to T
+// on load): the raw blending factors of shock capturing (into alpha_in, unless
+// they are there), the outer states of Dirichlet boundaries, and the fluxes of
+// slip walls and mortars.
+template <typename T, typename S>
+int launch_before_element(trixi_hip_ctx *ctx, const S *u, double t, const double *tdev, double *alpha_in,
+                          bool alpha_ready) {
   // shock capturing: raw indicator first (needs the whole state), smoothing
-  // happens inline. A stage reads the factors of state buffer par, computed by
-  // the previous fused stage when fresh.
-  const bool hg = is_hg(ctx);
-  double *alpha_in = so ? ctx->d_alpha_st[ctx->par] : ctx->d_alpha_raw;
-  if (hg) {
-    if (!(so && ctx->alpha_fresh)) {
+  // happens inline
+  if (is_hg(ctx)) {
+    if (!alpha_ready) {
       int r = launch_indicator_raw<T>(ctx, u, alpha_in);
       if (r) return r;
     }
@@ -581,7 +583,7 @@ int launch_rhs_T(trixi_hip_ctx *ctx, T *du, const T *u, double t, const double *
     bool ok = dispatch_dn(ctx->D, ctx->N, [&](auto Dc, auto Nc) {
       constexpr int D = decltype(Dc)::value, N = decltype(Nc)::value;
       const int total = ctx->B * ipow_c(N + 1, D - 1);
-      hipLaunchKernelGGL((slip_wall_flux_kernel<T, D, N>), dim3((total + 255) / 256), dim3(256), 0, ctx->stream, u,
+      hipLaunchKernelGGL((slip_wall_flux_kernel<T, D, N, S>), dim3((total + 255) / 256), dim3(256), 0, ctx->stream, u,
                          ctx->d_bnd, ctx->B, ctx->cfg.gamma, (T *)ctx->d_mflux);
     });
     if (!ok) return TRIXI_HIP_EINVAL;
@@ -590,7 +592,7 @@ int launch_rhs_T(trixi_hip_ctx *ctx, T *du, const T *u, double t, const double *
   if (ctx->M > 0) {  // fluxes of the mortar faces
     bool ok = dispatch_dn(ctx->D, ctx->N, [&](auto Dc, auto Nc) {
       constexpr int D = decltype(Dc)::value, N = decltype(Nc)::value;
-      constexpr int n = N + 1, S = 1 << (D - 1), TPM = S * (D == 3 ? n * n : n), MPB = 256 / TPM;
+      constexpr int n = N + 1, TPM = (1 << (D - 1)) * (D == 3 ? n * n : n), MPB = 256 / TPM;
       MortarConst<T, N> mc{};
       for (int i = 0; i < n * n; ++i) {
         mc.fu[i] = T(ctx->mfu[i]);
@@ -598,13 +600,30 @@ int launch_rhs_T(trixi_hip_ctx *ctx, T *du, const T *u, double t, const double *
         mc.ru[i] = T(ctx->mru[i]);
         mc.rl[i] = T(ctx->mrl[i]);
       }
-      hipLaunchKernelGGL((mortar_flux_kernel<T, D, N>), dim3((ctx->M + MPB - 1) / MPB), dim3(256), 0, ctx->stream,
+      hipLaunchKernelGGL((mortar_flux_kernel<T, D, N, S>), dim3((ctx->M + MPB - 1) / MPB), dim3(256), 0, ctx->stream,
                          u, ctx->d_mort, ctx->M, ctx->B, ctx->cfg.surface_flux, T(ctx->cfg.gamma), mc,
                          (T *)ctx->d_mflux);
     });
     if (!ok) return TRIXI_HIP_EINVAL;
     HIP_TRY(hipGetLastError());
   }
+  return TRIXI_HIP_OK;
+}
+
+// The RHS of u into du, or (so) a fused 2N stage. FP32 only: with u64 != null the
+// RHS of the FP64 array u64 (rounded on load) instead of u, with du64 != null
+// into the FP64 array du64 instead of du.
+template <typename T>
+int launch_rhs_T(trixi_hip_ctx *ctx, T *du, const T *u, double t, const double *tdev,
+                 const StageOut *so = nullptr, const double *u64 = nullptr, double *du64 = nullptr) {
+  // A stage reads the factors of state buffer par, computed by the previous
+  // fused stage when fresh.
+  const bool hg = is_hg(ctx);
+  double *alpha_in = so ? ctx->d_alpha_st[ctx->par] : ctx->d_alpha_raw;
+  const bool alpha_ready = so && ctx->alpha_fresh;
+  int rb = u64 ? launch_before_element<T>(ctx, u64, t, tdev, alpha_in, alpha_ready)
+               : launch_before_element<T>(ctx, u, t, tdev, alpha_in, alpha_ready);
+  if (rb) return rb;
   ElemArgs<T> a{};
   a.u = u;
   a.du = du;
@@ -644,10 +663,15 @@ int launch_rhs_T(trixi_hip_ctx *ctx, T *du, const T *u, double t, const double *
                          nullptr);
     }
   }
+  if (u64) a.u64 = u64;
+  a.du64 = du64;
   a.gamma64 = ctx->cfg.gamma;
   const int epb = so ? ctx->epb_st : ctx->epb;
   int nblocks = (ctx->E + epb - 1) / epb;
-  hipError_t e = (so ? ctx->elem_stage : ctx->elem)(&a, ctx->kconst.data(), nblocks, ctx->stream);
+  ElemLaunch launch = so ? ctx->elem_stage : ctx->elem;
+  if (du64 && !(launch = find_launch(ctx, ELEM_RHS64, ctx->epb, ctx->nt)))
+    return set_err(ctx, TRIXI_HIP_EINVAL, "no element kernel between FP64 arrays for this tile");
+  hipError_t e = launch(&a, ctx->kconst.data(), nblocks, ctx->stream);
   if (e != hipSuccess) return set_err(ctx, TRIXI_HIP_EHIP, std::string("element kernel launch: ") + hipGetErrorString(e));
   return TRIXI_HIP_OK;
 }
@@ -1020,8 +1044,7 @@ int trixi_hip_create(const trixi_hip_config *cfg, const trixi_hip_mesh *mesh,
          dev_alloc(ctx, &ctx->d_adj, std::max<size_t>(adj.size(), 1) * 4) == hipSuccess;
   if (ok && ctx->fp32)
     ok = dev_alloc(ctx, &ctx->d_u32b[0], nv * 4) == hipSuccess && dev_alloc(ctx, &ctx->d_u32b[1], nv * 4) == hipSuccess &&
-         dev_alloc(ctx, &ctx->d_su32, nv * 4) == hipSuccess &&
-         dev_alloc(ctx, &ctx->d_sdu32, nv * 4) == hipSuccess;
+         dev_alloc(ctx, &ctx->d_su32, nv * 4) == hipSuccess;
   if (!ok) {
     trixi_hip_destroy(ctx);
     fprintf(stderr, "trixi_hip_create: device allocation failed\n");
@@ -1073,7 +1096,7 @@ int trixi_hip_destroy(trixi_hip_ctx *ctx) {
   drop_graphs(ctx);
   void *ptrs[] = {ctx->d_nbr, ctx->d_invj, ctx->d_centers, ctx->d_ub[0], ctx->d_ub[1], ctx->d_utmp,
                   ctx->d_u32b[0], ctx->d_u32b[1], ctx->d_du,
-                  ctx->d_hu, ctx->d_hdu, ctx->d_su32, ctx->d_sdu32, ctx->d_alpha_raw, ctx->d_alpha,
+                  ctx->d_hu, ctx->d_hdu, ctx->d_su32, ctx->d_alpha_raw, ctx->d_alpha,
                   ctx->d_alpha_st[0], ctx->d_alpha_st[1],
                   ctx->d_partial, ctx->d_scalars, ctx->d_mlp, ctx->d_feat, ctx->d_mlp_partial,
                   ctx->d_alpha_hg, ctx->d_mlp_img, ctx->d_records, ctx->d_bx, ctx->d_ghost, ctx->d_mort,
@@ -1161,9 +1184,13 @@ int trixi_hip_rhs(trixi_hip_ctx *ctx, double *du, const double *u, double t, int
   }
   int r;
   if (ctx->fp32) {
-    if ((r = convert<float, double>(ctx, ctx->d_su32, du_in, nv))) return r;
-    if ((r = launch_rhs_T<float>(ctx, ctx->d_sdu32, ctx->d_su32, t, nullptr))) return r;
-    if ((r = convert<double, float>(ctx, du_out, ctx->d_sdu32, nv))) return r;
+    // one launch between the FP64 arrays; where they overlap, elements would read
+    // neighbours that others have already overwritten: from a rounded copy then
+    const bool overlap = (uintptr_t)du_out < (uintptr_t)(du_in + nv) && (uintptr_t)du_in < (uintptr_t)(du_out + nv);
+    if (overlap && (r = convert<float, double>(ctx, ctx->d_su32, du_in, nv))) return r;
+    if ((r = launch_rhs_T<float>(ctx, nullptr, overlap ? ctx->d_su32 : nullptr, t, nullptr, nullptr,
+                                 overlap ? nullptr : du_in, du_out)))
+      return r;
   } else {
     if ((r = launch_rhs_T<double>(ctx, du_out, du_in, t, nullptr))) return r;
   }
@@ -1966,7 +1993,7 @@ int trixi_hip_autotune(trixi_hip_ctx *ctx, int repetitions, trixi_hip_tile_timin
   for (const auto &kv : elem_registry()) {
     const ElemKey &k = kv.first;
     if (k.fp32 == (ctx->fp32 ? 1 : 0) && k.D == ctx->D && k.N == ctx->N && k.vol == ctx->vol &&
-        k.bnd == (ctx->B + ctx->M > 0 ? 1 : 0) && (k.stage == 0 || fused))
+        k.bnd == (ctx->B + ctx->M > 0 ? 1 : 0) && (k.stage == ELEM_RHS || (k.stage == ELEM_STAGE && fused)))
       cand.push_back(Cand{k.stage, k.epb, k.nt, kv.second, 1e300});
   }
   // captured steps hold the kernels of the old tiles
