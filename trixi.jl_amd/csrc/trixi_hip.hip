@@ -96,6 +96,8 @@ template <typename F> bool dispatch_dn(int D, int N, F &&f) {
 
 constexpr int kMaxPartials = 1 << 16;
 constexpr int kMaxSpeedBlocks = 1 << 16;  // workgroups (and partials) of the wave-speed reduction
+constexpr int kAnalysisBlocks = 1024;  // workgroups of the error norms; twice as many of the integrals
+static_assert(2 * kAnalysisBlocks * 10 <= kMaxPartials, "their partial results fit");
 constexpr int kMlpMaxWaves = 1024;  // partial gradient rows of one training step
 constexpr int kEagerSolveSteps = 8;  // trixi_hip_solve with at most this many steps launches without graphs
 
@@ -1305,7 +1307,7 @@ int total_volumes(trixi_hip_ctx *ctx) {
 // -> out[0, 2V): {sum w J (u - u_exact)^2 [V], max |u - u_exact| [V]}.
 int enqueue_error_sums(trixi_hip_ctx *ctx, double t, const double *tdev, double *out) {
   const int V = ctx->V, E = ctx->E;
-  if ((size_t)E * 2 * V > ctx->partial_cap) return set_err(ctx, TRIXI_HIP_EINVAL, "partials too small");
+  int blocks = 0;
   bool ok = dispatch_dn(ctx->D, ctx->N, [&](auto Dc, auto Nc) {
     constexpr int D = decltype(Dc)::value, N = decltype(Nc)::value;
     constexpr int NA = 2 * N + 1;
@@ -1313,12 +1315,18 @@ int enqueue_error_sums(trixi_hip_ctx *ctx, double t, const double *tdev, double 
     for (int i = 0; i < NA * (N + 1); ++i) ac.vdm[i] = ctx->a_vdm[i];
     for (int i = 0; i < NA; ++i) ac.aw[i] = ctx->a_weights[i];
     for (int i = 0; i <= N; ++i) ac.nodes[i] = ctx->nodes[i];
-    hipLaunchKernelGGL((error_norms_kernel<double, D, N, NA>), dim3(E), dim3(256), 0, ctx->stream, cur_u64(ctx),
-                       ctx->d_invj, ctx->d_centers, E, t, tdev, ctx->exact, ac, ctx->d_partial);
+    // as many tiles for each of up to kAnalysisBlocks workgroups (3 or 4 fit a CU)
+    const int tiles = (E + NormsTile<D, N>::EB - 1) / NormsTile<D, N>::EB;
+    const int each = (tiles + kAnalysisBlocks - 1) / kAnalysisBlocks;
+    blocks = (tiles + each - 1) / each;
+    hipLaunchKernelGGL((plain_exact(ctx->exact) ? error_norms_kernel<D, N, true> : error_norms_kernel<D, N, false>),
+                       dim3(blocks), dim3(256), 0, ctx->stream, cur_u64(ctx), ctx->d_invj, ctx->d_centers, E, t, tdev,
+                       ctx->exact, ac, ctx->d_partial);
   });
   if (!ok) return TRIXI_HIP_EINVAL;
   HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(reduce_columns_kernel, dim3(1), dim3(256), 0, ctx->stream, ctx->d_partial, E, 2 * V, V, out);
+  hipLaunchKernelGGL(reduce_columns_kernel, dim3(2 * V), dim3(256), 0, ctx->stream, ctx->d_partial, blocks, 2 * V, V,
+                     out);
   HIP_TRY(hipGetLastError());
   return TRIXI_HIP_OK;
 }
@@ -1326,16 +1334,16 @@ int enqueue_error_sums(trixi_hip_ctx *ctx, double t, const double *tdev, double 
 // integrate_via_indices sums of u and the mathematical entropy -> out[0, V + 1).
 int enqueue_integral_sums(trixi_hip_ctx *ctx, double *out) {
   const int V = ctx->V, E = ctx->E;
-  if ((size_t)E * (V + 1) > ctx->partial_cap) return set_err(ctx, TRIXI_HIP_EINVAL, "partials too small");
+  const int blocks = (int)std::min<size_t>(((size_t)E * ctx->NN + 255) / 256, 2 * kAnalysisBlocks);
   bool ok = dispatch_dn(ctx->D, ctx->N, [&](auto Dc, auto Nc) {
     constexpr int D = decltype(Dc)::value, N = decltype(Nc)::value;
-    hipLaunchKernelGGL((integrals_kernel<double, D, N>), dim3((E + 255) / 256), dim3(256), 0, ctx->stream,
-                       cur_u64(ctx), ctx->d_invj, E, ctx->cfg.gamma, ctx->d_scalars + kWeights, ctx->d_partial);
+    hipLaunchKernelGGL((integrals_kernel<D, N>), dim3(blocks), dim3(256), 0, ctx->stream, cur_u64(ctx), ctx->d_invj, E,
+                       ctx->cfg.gamma, ctx->d_scalars + kWeights, ctx->d_partial);
   });
   if (!ok) return TRIXI_HIP_EINVAL;
   HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(reduce_columns_kernel, dim3(1), dim3(256), 0, ctx->stream, ctx->d_partial, E, V + 1, V + 1,
-                     out);
+  hipLaunchKernelGGL(reduce_columns_kernel, dim3(V + 1), dim3(256), 0, ctx->stream, ctx->d_partial, blocks, V + 1,
+                     V + 1, out);
   HIP_TRY(hipGetLastError());
   return TRIXI_HIP_OK;
 }
