@@ -66,12 +66,11 @@ __device__ __forceinline__ f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
-// BF16 weight images in LDS: W1 [NH][KF] (features padded with zeros), W2
-// [NH][NH] and its transpose.
+// BF16 weight images in LDS: W1 [NH][KF] (features padded with zeros) and W2
+// [NH][NH].
 struct WeightsLDS {
   uint16_t w1[NH * KF];
   uint16_t w2[NH * NH];
-  uint16_t w2t[NH * NH];
   float b1[NH], b2[NH], w3[NH], b3;
 };
 
@@ -80,12 +79,7 @@ __device__ __forceinline__ void load_weights(const float *__restrict__ w, Weight
     const int h = i / KF, f = i - h * KF;
     s.w1[i] = f < NF ? to_bf16(w[OFF_W1 + h * NF + f]) : 0;
   }
-  for (int i = threadIdx.x; i < NH * NH; i += blockDim.x) {
-    const int o = i / NH, in = i - o * NH;
-    const uint16_t v = to_bf16(w[OFF_W2 + i]);
-    s.w2[i] = v;
-    s.w2t[in * NH + o] = v;
-  }
+  for (int i = threadIdx.x; i < NH * NH; i += blockDim.x) s.w2[i] = to_bf16(w[OFF_W2 + i]);
   for (int i = threadIdx.x; i < NH; i += blockDim.x) {
     s.b1[i] = w[OFF_B1 + i];
     s.b2[i] = w[OFF_B2 + i];
@@ -218,19 +212,17 @@ __device__ __forceinline__ void forward_layers_regs(const WeightRegs &w, Tile &t
   t.y = 1.f / (1.f + __expf(-o));
 }
 
-__device__ __forceinline__ void forward_tile(const float *__restrict__ x, int n, int tile, const WeightsLDS &s,
-                                             Tile &t) {
+// X^T as the B operand: element l % 16 of the tile, features kb * 16 + 4 (l / 16) + j
+__device__ __forceinline__ void load_tile(const float *__restrict__ x, int n, int tile, Tile &t) {
   const int l = threadIdx.x & 63;
   const int e = tile * 16 + (l & 15);
   const int g = l >> 4;
-  // X^T as the B operand: element e, features kb*16 + 4g + j
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb) {
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (e < n) v = *reinterpret_cast<const float4 *>(x + (size_t)e * KF + kb * 16 + 4 * g);
     t.xb[kb] = pack4(v.x, v.y, v.z, v.w);
   }
-  forward_layers(s, t);
 }
 
 // The network as inference reads it: BF16 images of W1 (features padded with
@@ -245,6 +237,40 @@ struct InferImage {
   float b1[NH], b2[NH], w3[NH], b3, pad[3];
 };
 static_assert(sizeof(InferImage) % 16 == 0, "16-byte copies");
+
+// With the transpose of W2 beside it, in the same fragment order (lane l: input row
+// 16 ib + l % 16, outputs 16 ob + 4 (l / 16) + 0..3), which the gradient needs.
+struct TrainImage {
+  InferImage infer;
+  uint16_t w2tf[4 * 4 * 64 * 4];
+};
+
+// Index of (row, k) in a fragment-ordered image with KB blocks of 16 along k.
+template <int KB> __host__ __device__ constexpr int frag_index(int row, int k) {
+  return (((row >> 4) * KB + (k >> 4)) * 64 + (row & 15) + 16 * ((k & 15) >> 2)) * 4 + (k & 3);
+}
+
+// Parameter p of the FP32 vector, of value w, into the images (the padded
+// features of W1 stay as mlp_pack_kernel wrote them).
+__device__ __forceinline__ void pack_param(TrainImage &img, int p, float w) {
+  if (p < OFF_B1) {
+    const int h = p / NF;
+    img.infer.w1f[frag_index<2>(h, p - h * NF)] = to_bf16(w);
+  } else if (p < OFF_W2) {
+    img.infer.b1[p - OFF_B1] = w;
+  } else if (p < OFF_B2) {
+    const int o = (p - OFF_W2) / NH, in = (p - OFF_W2) % NH;
+    const uint16_t h = to_bf16(w);
+    img.infer.w2f[frag_index<4>(o, in)] = h;
+    img.w2tf[frag_index<4>(in, o)] = h;
+  } else if (p < OFF_W3) {
+    img.infer.b2[p - OFF_B2] = w;
+  } else if (p < OFF_B3) {
+    img.infer.w3[p - OFF_W3] = w;
+  } else {
+    img.infer.b3 = w;
+  }
+}
 
 __device__ __forceinline__ bf16x4 frag_w1(const InferImage &s, int hb, int kb) {
   return lds4(&s.w1f[((hb * 2 + kb) * 64 + (threadIdx.x & 63)) * 4]);

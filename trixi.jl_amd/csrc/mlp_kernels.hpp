@@ -9,28 +9,14 @@
 namespace trixi_hip {
 namespace mlp {
 
-// FP32 parameters -> InferImage (one workgroup).
-__global__ __launch_bounds__(256) void mlp_pack_kernel(const float *__restrict__ w, InferImage *__restrict__ img) {
-  for (int i = threadIdx.x; i < NH; i += blockDim.x) {
-    img->b1[i] = w[OFF_B1 + i];
-    img->b2[i] = w[OFF_B2 + i];
-    img->w3[i] = w[OFF_W3 + i];
-  }
-  if (threadIdx.x == 0) {
-    img->b3 = w[OFF_B3];
-    img->pad[0] = img->pad[1] = img->pad[2] = 0.f;
-  }
-  // W1 and W2 in fragment order: [block][kb][lane][4]
-  for (int i = threadIdx.x; i < 4 * 2 * 64 * 4; i += blockDim.x) {
-    const int jj = i & 3, l = (i >> 2) & 63, kb = (i >> 8) & 1, hb = i >> 9;
-    const int h = hb * 16 + (l & 15), f = kb * 16 + 4 * (l >> 4) + jj;
-    img->w1f[i] = f < NF ? to_bf16(w[OFF_W1 + h * NF + f]) : 0;
-  }
-  for (int i = threadIdx.x; i < 4 * 4 * 64 * 4; i += blockDim.x) {
-    const int jj = i & 3, l = (i >> 2) & 63, kb = (i >> 8) & 3, ob = i >> 10;
-    const int o = ob * 16 + (l & 15), k = kb * 16 + 4 * (l >> 4) + jj;
-    img->w2f[i] = to_bf16(w[OFF_W2 + o * NH + k]);
-  }
+// FP32 parameters -> images (one thread for each parameter, then the padded features).
+constexpr int PACK_BLOCKS = (NP + NH * (KF - NF) + 255) / 256;
+__global__ __launch_bounds__(256) void mlp_pack_kernel(const float *__restrict__ w, TrainImage *__restrict__ img) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  const int i = p - NP;
+  if (p < NP) pack_param(*img, p, w[p]);
+  else if (i < NH * (KF - NF)) img->infer.w1f[frag_index<2>(i / (KF - NF), NF + i % (KF - NF))] = 0;
+  if (p < 3) img->infer.pad[p] = 0.f;
 }
 
 // Inference over E elements: alpha_raw[e] = hg_clip(alpha_max * y(features[e])),
@@ -49,7 +35,8 @@ __global__ __launch_bounds__(NTHR) void mlp_infer_kernel(const float *__restrict
   const int ntiles = (E + 15) / 16;
   for (int tile = blockIdx.x * WAVES + wave; tile < ntiles; tile += gridDim.x * WAVES) {
     Tile t;
-    forward_tile(x, E, tile, s, t);
+    load_tile(x, E, tile, t);
+    forward_layers(s, t);
     const int e = tile * 16 + l;
     if (l < 16 && e < E) {
       if (y_out) y_out[e] = t.y;
@@ -68,25 +55,51 @@ __global__ __launch_bounds__(NTHR) void mlp_infer_kernel(const float *__restrict
   }
 }
 
+// Sum over the 16 lanes of a row group, in every lane: the pairs of a butterfly
+// over lane bits 0..3 in DPP moves (quads, then mirrored halves and rows: after
+// two steps the lanes of a quad agree, so a mirrored lane holds what the lane with
+// one bit flipped does).
+template <int CTRL> __device__ __forceinline__ float dpp_move(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row_sum(float x) {
+  x += dpp_move<0xB1>(x);   // quad_perm 1 0 3 2
+  x += dpp_move<0x4E>(x);   // quad_perm 2 3 0 1
+  x += dpp_move<0x141>(x);  // row_half_mirror
+  x += dpp_move<0x140>(x);  // row_mirror
+  return x;
+}
+
 // Loss L = sum_e (y_e - target_e)^2 / n and its gradient. Each wavefront
 // handles tiles w, w + W, ... and writes one partial row [NPL] (gradient,
-// then loss) to partial[global wave]; mlp_reduce_kernel sums the rows.
-__global__ __launch_bounds__(NTHR) void mlp_grad_kernel(const float *__restrict__ w, const float *__restrict__ x,
-                                                        const float *__restrict__ target, int n,
-                                                        float *__restrict__ partial) {
-  __shared__ __attribute__((aligned(16))) WeightsLDS s;
-  // per-wave transposes [hidden or feature][element], BF16
-  __shared__ __attribute__((aligned(16))) uint16_t s_x[WAVES][KF * 16];
-  __shared__ __attribute__((aligned(16))) uint16_t s_h1[WAVES][NH * 16];
-  __shared__ __attribute__((aligned(16))) uint16_t s_d2[WAVES][NH * 16];
-  __shared__ __attribute__((aligned(16))) uint16_t s_d1[WAVES][NH * 16];
-  load_weights(w, s);
-  __syncthreads();
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
+// then loss) to partial[w]; mlp_reduce_kernel sums the rows.
+//
+// A minibatch has few tiles (512 of them at 8192 elements, two wavefronts for each
+// CU), so a launch lasts as long as one wavefront's chain. Hence one wavefront for each
+// workgroup, spread over all CUs, with the weights loaded as fragments from the
+// image into registers, all at once: 25.5 us with
+// four wavefronts to a workgroup that converted the FP32 weights into LDS first,
+// 13.9 us now (8192 elements).
+__global__ __launch_bounds__(64) void mlp_grad_kernel(const TrainImage *__restrict__ img, const float *__restrict__ x,
+                                                      const float *__restrict__ target, int n,
+                                                      float *__restrict__ partial) {
+  // transposes [hidden or feature][element], BF16
+  __shared__ __attribute__((aligned(16))) uint16_t s_x[KF * 16];
+  __shared__ __attribute__((aligned(16))) uint16_t s_h1[NH * 16];
+  __shared__ __attribute__((aligned(16))) uint16_t s_d2[NH * 16];
+  __shared__ __attribute__((aligned(16))) uint16_t s_d1[NH * 16];
+  const int l = threadIdx.x;
   const int g = l >> 4, c = l & 15;
-  const int gw = blockIdx.x * WAVES + wave, nw = gridDim.x * WAVES;
+  const int gw = blockIdx.x, nw = gridDim.x;
   const int ntiles = (n + 15) / 16;
   const float inv_n = 1.f / (float)n;
+  WeightRegs wr;
+  load_weight_regs(img->infer, wr);
+  bf16x4 w2t[4][4];
+#pragma unroll
+  for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) w2t[ib][ob] = lds4(&img->w2tf[((ib * 4 + ob) * 64 + l) * 4]);
 
   f32x4 gW1[4][2], gW2[4][4];
 #pragma unroll
@@ -103,10 +116,11 @@ __global__ __launch_bounds__(NTHR) void mlp_grad_kernel(const float *__restrict_
 
   for (int tile = gw; tile < ntiles; tile += nw) {
     Tile t;
-    forward_tile(x, n, tile, s, t);
+    load_tile(x, n, tile, t);
     const int e = tile * 16 + c;
     const bool ok = e < n;
     const float tgt = ok ? target[e] : 0.f;
+    forward_layers_regs(wr, t);
     const float res = ok ? t.y - tgt : 0.f;
     if (g == 0) {
       loss += res * res * inv_n;
@@ -119,10 +133,9 @@ __global__ __launch_bounds__(NTHR) void mlp_grad_kernel(const float *__restrict_
     for (int ob = 0; ob < 4; ++ob) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int h = ob * 16 + 4 * g + r;
         const float z = t.z2[ob][r];
         gw3[ob * 4 + r] += dout * (z > 0.f ? z : 0.f);
-        const float dz = z > 0.f ? s.w3[h] * dout : 0.f;
+        const float dz = z > 0.f ? wr.w3[ob][r] * dout : 0.f;
         d2[ob][r] = dz;
         gb2[ob * 4 + r] += dz;
       }
@@ -136,7 +149,7 @@ __global__ __launch_bounds__(NTHR) void mlp_grad_kernel(const float *__restrict_
     for (int ib = 0; ib < 4; ++ib) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ob = 0; ob < 4; ++ob) acc = mfma(lds4(&s.w2t[(ib * 16 + c) * NH + ob * 16 + 4 * g]), d2b[ob], acc);
+      for (int ob = 0; ob < 4; ++ob) acc = mfma(w2t[ib][ob], d2b[ob], acc);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float dz = t.z1[ib][r] > 0.f ? acc[r] : 0.f;
@@ -148,31 +161,31 @@ __global__ __launch_bounds__(NTHR) void mlp_grad_kernel(const float *__restrict_
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s_x[wave][(kb * 16 + 4 * g + j) * 16 + c] = (uint16_t)t.xb[kb][j];
+      for (int j = 0; j < 4; ++j) s_x[(kb * 16 + 4 * g + j) * 16 + c] = (uint16_t)t.xb[kb][j];
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int row = (b * 16 + 4 * g + j) * 16 + c;
-        s_h1[wave][row] = (uint16_t)t.h1b[b][j];
-        s_d2[wave][row] = (uint16_t)d2b[b][j];
-        s_d1[wave][row] = to_bf16(d1[b][j]);
+        s_h1[row] = (uint16_t)t.h1b[b][j];
+        s_d2[row] = (uint16_t)d2b[b][j];
+        s_d1[row] = to_bf16(d1[b][j]);
       }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     // dW2 (out x in) += dZ2^T H1: A = dZ2^T rows, B = H1 columns, K = element
 #pragma unroll
     for (int ob = 0; ob < 4; ++ob) {
-      const bf16x4 a = lds4(&s_d2[wave][(ob * 16 + c) * 16 + 4 * g]);
+      const bf16x4 a = lds4(&s_d2[(ob * 16 + c) * 16 + 4 * g]);
 #pragma unroll
-      for (int ib = 0; ib < 4; ++ib) gW2[ob][ib] = mfma(a, lds4(&s_h1[wave][(ib * 16 + c) * 16 + 4 * g]), gW2[ob][ib]);
+      for (int ib = 0; ib < 4; ++ib) gW2[ob][ib] = mfma(a, lds4(&s_h1[(ib * 16 + c) * 16 + 4 * g]), gW2[ob][ib]);
     }
     // dW1 (hidden x feature) += dZ1^T X
 #pragma unroll
     for (int hb = 0; hb < 4; ++hb) {
-      const bf16x4 a = lds4(&s_d1[wave][(hb * 16 + c) * 16 + 4 * g]);
+      const bf16x4 a = lds4(&s_d1[(hb * 16 + c) * 16 + 4 * g]);
 #pragma unroll
-      for (int fb = 0; fb < 2; ++fb) gW1[hb][fb] = mfma(a, lds4(&s_x[wave][(fb * 16 + c) * 16 + 4 * g]), gW1[hb][fb]);
+      for (int fb = 0; fb < 2; ++fb) gW1[hb][fb] = mfma(a, lds4(&s_x[(fb * 16 + c) * 16 + 4 * g]), gW1[hb][fb]);
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -181,18 +194,12 @@ __global__ __launch_bounds__(NTHR) void mlp_grad_kernel(const float *__restrict_
   // per-lane vectors summed over the 16 lanes of a row group (elements)
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) {
-      gb1[i] += __shfl_xor(gb1[i], m);
-      gb2[i] += __shfl_xor(gb2[i], m);
-      gw3[i] += __shfl_xor(gw3[i], m);
-    }
+    gb1[i] = row_sum(gb1[i]);
+    gb2[i] = row_sum(gb2[i]);
+    gw3[i] = row_sum(gw3[i]);
   }
-#pragma unroll
-  for (int m = 1; m < 16; m <<= 1) {
-    gb3 += __shfl_xor(gb3, m);
-    loss += __shfl_xor(loss, m);
-  }
+  gb3 = row_sum(gb3);
+  loss = row_sum(loss);
   float *row = partial + (size_t)gw * NPL;
   // accumulator layout: row 4g + r, column c of each 16 x 16 tile
 #pragma unroll
@@ -229,17 +236,47 @@ __global__ __launch_bounds__(NTHR) void mlp_grad_kernel(const float *__restrict_
 // workgroup takes RED_COLS consecutive columns; its RED_SPLIT row groups sum
 // rows g, g + RED_SPLIT, ... in row order (each load instruction of a
 // wavefront reads two rows of 32 consecutive columns), then the group sums are
-// added in group order. Deterministic, and RED_SPLIT independent load streams
-// per column instead of one serial chain over all rows.
-constexpr int RED_COLS = 32, RED_SPLIT = 8;
+// added in group order. Bound by the latency of the rows, which other XCDs wrote:
+// RED_BATCH loads are in flight at a time (rows past the end add +0, which
+// leaves a sum that began at +0 as it is).
+//
+// STEP: also one Adam step (Kingma & Ba 2015; step = 1, 2, ...) on the FP32 master
+// weights w with the moments m and v, and the new weight into the images, by the
+// thread that holds the gradient's sum. As four launches (reduction with two
+// loads in flight, Adam, packing by one workgroup) a training step on 8192
+// elements took 58 us, with this 24.
+constexpr int RED_COLS = 32, RED_SPLIT = 8, RED_BATCH = 32;
+struct AdamArgs {
+  float *w, *m, *v;
+  TrainImage *img;
+  float lr, beta1, beta2, eps;
+  int step;
+};
+template <bool STEP>
 __global__ __launch_bounds__(RED_COLS *RED_SPLIT) void mlp_reduce_kernel(const float *__restrict__ partial, int rows,
-                                                                         float *__restrict__ out) {
+                                                                         float *__restrict__ out, AdamArgs a) {
   __shared__ float s_part[RED_SPLIT][RED_COLS];
   const int c = threadIdx.x % RED_COLS, g = threadIdx.x / RED_COLS;
   const int p = blockIdx.x * RED_COLS + c;
+  float mi = 0.f, vi = 0.f, wi = 0.f;
+  if (STEP && g == 0 && p < NP) {
+    mi = a.m[p];
+    vi = a.v[p];
+    wi = a.w[p];
+  }
   float acc = 0.f;
-  if (p < NPL)
-    for (int r = g; r < rows; r += RED_SPLIT) acc += partial[(size_t)r * NPL + p];
+  if (p < NPL) {
+    for (int r0 = g; r0 < rows; r0 += RED_SPLIT * RED_BATCH) {
+      float x[RED_BATCH];
+#pragma unroll
+      for (int i = 0; i < RED_BATCH; ++i) {
+        const int r = r0 + RED_SPLIT * i;
+        x[i] = r < rows ? partial[(size_t)r * NPL + p] : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < RED_BATCH; ++i) acc += x[i];
+    }
+  }
   s_part[g][c] = acc;
   __syncthreads();
   if (g == 0 && p < NPL) {
@@ -247,23 +284,18 @@ __global__ __launch_bounds__(RED_COLS *RED_SPLIT) void mlp_reduce_kernel(const f
 #pragma unroll
     for (int k = 1; k < RED_SPLIT; ++k) t += s_part[k][c];
     out[p] = t;
+    if (STEP && p < NP) {
+      mi = a.beta1 * mi + (1.f - a.beta1) * t;
+      vi = a.beta2 * vi + (1.f - a.beta2) * t * t;
+      a.m[p] = mi;
+      a.v[p] = vi;
+      const float mh = mi / (1.f - powf(a.beta1, (float)a.step));
+      const float vh = vi / (1.f - powf(a.beta2, (float)a.step));
+      wi -= a.lr * mh / (sqrtf(vh) + a.eps);
+      a.w[p] = wi;
+      pack_param(*a.img, p, wi);
+    }
   }
-}
-
-// Adam (Kingma & Ba 2015) on the FP32 master weights; step = 1, 2, ...
-__global__ __launch_bounds__(256) void mlp_adam_kernel(float *__restrict__ w, float *__restrict__ m,
-                                                       float *__restrict__ v, const float *__restrict__ grad, float lr,
-                                                       float beta1, float beta2, float eps, int step) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= NP) return;
-  const float gr = grad[p];
-  const float mi = beta1 * m[p] + (1.f - beta1) * gr;
-  const float vi = beta2 * v[p] + (1.f - beta2) * gr * gr;
-  m[p] = mi;
-  v[p] = vi;
-  const float mh = mi / (1.f - powf(beta1, (float)step));
-  const float vh = vi / (1.f - powf(beta2, (float)step));
-  w[p] -= lr * mh / (sqrtf(vh) + eps);
 }
 
 }  // namespace mlp

@@ -201,7 +201,7 @@ struct trixi_hip_ctx {
   // learned indicator (2D p3): d_mlp = weights [NP] | Adam m [NP] | Adam v [NP]
   // | feature box lo [NF] | hi [NF] | gradient + loss [NPL]
   float *d_mlp = nullptr, *d_feat = nullptr, *d_mlp_partial = nullptr;
-  mlp::InferImage *d_mlp_img = nullptr;  // BF16 inference image of the parameters
+  mlp::TrainImage *d_mlp_img = nullptr;  // BF16 images of the parameters
   double *d_alpha_hg = nullptr;
   bool mlp_ready = false;
   int mlp_step = 0;
@@ -465,7 +465,7 @@ Ind2DArgs ind2d_args(const trixi_hip_ctx *ctx, const HGParams &params, bool net,
   Ind2DArgs ia{};
   ia.hp = params;
   for (int i = 0; i < 16; ++i) ia.vi.v[i] = ctx->Vinv[i];
-  ia.img = ctx->d_mlp_img;
+  ia.img = ctx->d_mlp_img ? &ctx->d_mlp_img->infer : nullptr;
   ia.lo = ctx->d_mlp ? ctx->d_mlp + 3 * mlp::NP : nullptr;
   ia.hi = ctx->d_mlp ? ia.lo + mlp::NF : nullptr;
   ia.net = net ? 1 : 0;
@@ -518,11 +518,9 @@ int launch_hg(trixi_hip_ctx *ctx, const S *u, double *alpha_out, float *feat, co
   return TRIXI_HIP_OK;
 }
 
-int mlp_blocks(int n) {
-  const int ntiles = (n + 15) / 16;
-  const int waves = std::min(std::max(ntiles, 1), kMlpMaxWaves);
-  return (waves + mlp::WAVES - 1) / mlp::WAVES;
-}
+// wavefronts of a launch over n elements (16 to a tile)
+int mlp_waves(int n) { return std::min(std::max((n + 15) / 16, 1), kMlpMaxWaves); }
+int mlp_blocks(int n) { return (mlp_waves(n) + mlp::WAVES - 1) / mlp::WAVES; }
 
 // Raw (unsmoothed) blending factors of state u into alpha_out, from the
 // indicator selected by ind_mode.
@@ -1646,14 +1644,14 @@ static int mlp_check(trixi_hip_ctx *ctx) {
   HIP_TRY(dev_alloc(ctx, &ctx->d_feat, (size_t)ctx->E * kMlpFeatureStride * 4));
   HIP_TRY(dev_alloc(ctx, &ctx->d_alpha_hg, (size_t)ctx->E * 8));
   HIP_TRY(dev_alloc(ctx, &ctx->d_mlp_partial, (size_t)kMlpMaxWaves * mlp::NPL * 4));
-  HIP_TRY(dev_alloc(ctx, &ctx->d_mlp_img, sizeof(mlp::InferImage)));
+  HIP_TRY(dev_alloc(ctx, &ctx->d_mlp_img, sizeof(mlp::TrainImage)));
   return TRIXI_HIP_OK;
 }
 
-// Refresh the BF16 inference image after the parameters changed.
+// Refresh the BF16 images after the parameters were set.
 static int mlp_pack(trixi_hip_ctx *ctx) {
   ctx->alpha_fresh = false;  // the learned factors change with the parameters
-  hipLaunchKernelGGL(mlp::mlp_pack_kernel, dim3(1), dim3(256), 0, ctx->stream, ctx->d_mlp, ctx->d_mlp_img);
+  hipLaunchKernelGGL(mlp::mlp_pack_kernel, dim3(mlp::PACK_BLOCKS), dim3(256), 0, ctx->stream, ctx->d_mlp, ctx->d_mlp_img);
   HIP_TRY(hipGetLastError());
   return TRIXI_HIP_OK;
 }
@@ -1728,14 +1726,16 @@ int trixi_hip_mlp_forward(trixi_hip_ctx *ctx, const float *x_dev, int n, float *
   return TRIXI_HIP_OK;
 }
 
-static int mlp_gradient(trixi_hip_ctx *ctx, const float *x_dev, const float *target_dev, int n) {
-  const int nb = mlp_blocks(n);
-  hipLaunchKernelGGL(mlp::mlp_grad_kernel, dim3(nb), dim3(mlp::NTHR), 0, ctx->stream, ctx->d_mlp, x_dev, target_dev,
-                     n, ctx->d_mlp_partial);
+// Gradient and loss into the gradient buffer; with adam also the training step.
+static int mlp_gradient(trixi_hip_ctx *ctx, const float *x_dev, const float *target_dev, int n,
+                        const mlp::AdamArgs *adam) {
+  const int rows = mlp_waves(n);
+  hipLaunchKernelGGL(mlp::mlp_grad_kernel, dim3(rows), dim3(64), 0, ctx->stream, ctx->d_mlp_img, x_dev, target_dev, n,
+                     ctx->d_mlp_partial);
   HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(mlp::mlp_reduce_kernel, dim3((mlp::NPL + mlp::RED_COLS - 1) / mlp::RED_COLS),
-                     dim3(mlp::RED_COLS * mlp::RED_SPLIT), 0, ctx->stream, ctx->d_mlp_partial, nb * mlp::WAVES,
-                     mlp_grad_buffer(ctx));
+  hipLaunchKernelGGL(adam ? mlp::mlp_reduce_kernel<true> : mlp::mlp_reduce_kernel<false>,
+                     dim3((mlp::NPL + mlp::RED_COLS - 1) / mlp::RED_COLS), dim3(mlp::RED_COLS * mlp::RED_SPLIT), 0,
+                     ctx->stream, ctx->d_mlp_partial, rows, mlp_grad_buffer(ctx), adam ? *adam : mlp::AdamArgs{});
   HIP_TRY(hipGetLastError());
   return TRIXI_HIP_OK;
 }
@@ -1745,7 +1745,7 @@ int trixi_hip_mlp_loss_grad(trixi_hip_ctx *ctx, const float *x_dev, const float 
   if (!ctx || !x_dev || !target_dev || n <= 0) return TRIXI_HIP_EINVAL;
   if (!ctx->mlp_ready) return set_err(ctx, TRIXI_HIP_ESTATE, "no parameters set");
   if (((uintptr_t)x_dev & 15) != 0) return set_err(ctx, TRIXI_HIP_EINVAL, "features must be 16-byte aligned");
-  int r = mlp_gradient(ctx, x_dev, target_dev, n);
+  int r = mlp_gradient(ctx, x_dev, target_dev, n, nullptr);
   if (r) return r;
   if (grad_host)
     HIP_TRY(hipMemcpyAsync(grad_host, mlp_grad_buffer(ctx), mlp::NP * 4, hipMemcpyDeviceToHost, ctx->stream));
@@ -1759,14 +1759,12 @@ int trixi_hip_mlp_train_step(trixi_hip_ctx *ctx, const float *x_dev, const float
   if (!ctx || !x_dev || !target_dev || n <= 0 || !(learning_rate > 0.f)) return TRIXI_HIP_EINVAL;
   if (!ctx->mlp_ready) return set_err(ctx, TRIXI_HIP_ESTATE, "no parameters set");
   if (((uintptr_t)x_dev & 15) != 0) return set_err(ctx, TRIXI_HIP_EINVAL, "features must be 16-byte aligned");
-  int r = mlp_gradient(ctx, x_dev, target_dev, n);
+  ctx->alpha_fresh = false;  // the learned factors change with the parameters
+  const mlp::AdamArgs adam{ctx->d_mlp, ctx->d_mlp + mlp::NP, ctx->d_mlp + 2 * mlp::NP, ctx->d_mlp_img, learning_rate,
+                           0.9f,       0.999f,               1e-8f,                    ctx->mlp_step + 1};
+  int r = mlp_gradient(ctx, x_dev, target_dev, n, &adam);
   if (r) return r;
   ctx->mlp_step += 1;
-  hipLaunchKernelGGL(mlp::mlp_adam_kernel, dim3((mlp::NP + 255) / 256), dim3(256), 0, ctx->stream, ctx->d_mlp,
-                     ctx->d_mlp + mlp::NP, ctx->d_mlp + 2 * mlp::NP, mlp_grad_buffer(ctx), learning_rate, 0.9f,
-                     0.999f, 1e-8f, ctx->mlp_step);
-  HIP_TRY(hipGetLastError());
-  if ((r = mlp_pack(ctx))) return r;
   if (loss) {
     HIP_TRY(hipMemcpyAsync(loss, mlp_grad_buffer(ctx) + mlp::NP, 4, hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(host_sync(ctx));
