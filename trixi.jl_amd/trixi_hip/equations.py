@@ -277,7 +277,7 @@ initial_condition_weak_blast_wave = InitialCondition(
 def _ic_density_pulse(x, t, eq):
     # examples/tree_3d_dgsem/elixir_euler_amr.jl:15-26: a Gaussian density pulse
     # advected with v = 1 in every direction at p = 1
-    rho = 1 + np.exp(-np.sum(x ** 2, axis=-1)) / 2
+    rho = 1 + np.exp(-sum(x[..., d] ** 2 for d in range(eq.ndims))) / 2  # (np.sum over the short axis is slow)
     u = np.empty(x.shape[:-1] + (eq.nvariables(),))
     u[..., 0] = rho
     for d in range(eq.ndims):

@@ -79,30 +79,22 @@ class TreeMesh:
 
     def _build(self):
         D, L = self.ndims, self.initial_refinement_level
-        centers, icoords = [], []
-
-        def rec(level, center, length, ic):
-            if level >= L:
-                centers.append(center)
-                icoords.append(ic)
-                return
-            child_length = length / 2
-            for child in range(1 << D):
-                cc, ci = [], []
-                for d in range(D):
-                    sgn = 1 if (child >> d) & 1 else -1
-                    cc.append(center[d] + sgn * child_length / 2)
-                    ci.append(2 * ic[d] + (1 if sgn > 0 else 0))
-                rec(level + 1, tuple(cc), child_length, tuple(ci))
-
-        rec(0, self.center_level_0, self.length_level_0, (0,) * D)
+        # depth-first order is parent-major: a level's cells, each replaced by its
+        # children, whole levels at a time (one call per cell took 6.5 ms for 16^3)
+        side = np.array([[(child >> d) & 1 for d in range(D)] for child in range(1 << D)], dtype=np.int64)
+        centers = np.array([self.center_level_0], dtype=np.float64)  # [cells, D]
+        ic = np.zeros((1, D), dtype=np.int64)
+        child_length = self.length_level_0
+        for _ in range(L):
+            child_length = child_length / 2
+            centers = (centers[:, None, :] + (2 * side - 1) * child_length / 2).reshape(-1, D)
+            ic = (2 * ic[:, None, :] + side).reshape(-1, D)
         self.nelements = len(centers)
-        self.cell_centers = np.array(centers, dtype=np.float64)  # [E, D]
-        self._icoords = icoords
-        self._uniform_centers = self.cell_centers.copy()
+        self.cell_centers = centers  # [E, D]
+        self._icoords = ic
+        self._uniform_centers = centers.copy()
         self.cell_length = self.length_level_0 / (1 << L)
         nside = 1 << L
-        ic = np.array(icoords, dtype=np.int64)
         lin = np.zeros(self.nelements, dtype=np.int64)
         s = 1
         for d in range(D):
@@ -160,7 +152,7 @@ class TreeMesh:
         self._connect(nt)
 
     def _uniform_tree(self):
-        ic = np.array(self._icoords, dtype=np.int64).reshape(-1, self.ndims)
+        ic = self._icoords.copy()
         n = len(ic)
         return _Leaves(np.full(n, self.initial_refinement_level, np.int64), ic, self._uniform_centers.copy(),
                        np.zeros(n, np.int32), np.arange(n, dtype=np.int32))
