@@ -70,51 +70,47 @@ __device__ __forceinline__ float row_sum(float x) {
   return x;
 }
 
-// Loss L = sum_e (y_e - target_e)^2 / n and its gradient. Each wavefront
-// handles tiles w, w + W, ... and writes one partial row [NPL] (gradient,
-// then loss) to partial[w]; mlp_reduce_kernel sums the rows.
+// Loss L = sum_e (y_e - target_e)^2 / n and its gradient. Workgroup b of B
+// handles tiles b, b + B, ... and writes one partial row [NPL] (gradient, then
+// loss) to partial[b]; mlp_reduce_kernel sums the rows.
 //
-// A minibatch has few tiles (512 of them at 8192 elements, two wavefronts for each
-// CU), so a launch lasts as long as one wavefront's chain. Hence one wavefront for each
-// workgroup, spread over all CUs, with the weights loaded as fragments from the
-// image into registers, all at once: 25.5 us with
-// four wavefronts to a workgroup that converted the FP32 weights into LDS first,
-// 13.9 us now (8192 elements).
-__global__ __launch_bounds__(64) void mlp_grad_kernel(const TrainImage *__restrict__ img, const float *__restrict__ x,
-                                                      const float *__restrict__ target, int n,
-                                                      float *__restrict__ partial) {
-  // transposes [hidden or feature][element], BF16
-  __shared__ __attribute__((aligned(16))) uint16_t s_x[KF * 16];
-  __shared__ __attribute__((aligned(16))) uint16_t s_h1[NH * 16];
-  __shared__ __attribute__((aligned(16))) uint16_t s_d2[NH * 16];
-  __shared__ __attribute__((aligned(16))) uint16_t s_d1[NH * 16];
-  const int l = threadIdx.x;
+// A minibatch has few tiles (512 of them at 8192 elements), so a launch lasts as
+// long as one wavefront's chain of instructions and memory round trips. Hence four
+// wavefronts to a tile: each runs the forward pass, then wavefront w takes hidden rows
+// 16 w .. 16 w + 15 of both layers' gradients (and wavefront 0 the scalars). The
+// weights are loaded as fragments from the image into registers, all at once. 8192
+// elements: 25.2 us with one wavefront to a tile, four to a workgroup that converted
+// the FP32 weights into LDS first; 13.9 us with one, weights from the image; 12.1 us
+// with four, two tiles to a workgroup.
+__global__ __launch_bounds__(256) void mlp_grad_kernel(const TrainImage *__restrict__ img, const float *__restrict__ x,
+                                                       const float *__restrict__ target, int n,
+                                                       float *__restrict__ partial) {
+  // transposes [hidden or feature][element], BF16, of each wavefront
+  __shared__ __attribute__((aligned(16))) uint16_t s_x[4][KF * 16];
+  __shared__ __attribute__((aligned(16))) uint16_t s_h1[4][NH * 16];
+  __shared__ __attribute__((aligned(16))) uint16_t s_d2[4][16 * 16];
+  __shared__ __attribute__((aligned(16))) uint16_t s_d1[4][16 * 16];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
   const int g = l >> 4, c = l & 15;
-  const int gw = blockIdx.x, nw = gridDim.x;
   const int ntiles = (n + 15) / 16;
   const float inv_n = 1.f / (float)n;
   WeightRegs wr;
   load_weight_regs(img->infer, wr);
-  bf16x4 w2t[4][4];
+  bf16x4 w2t[4];  // of input rows 16 w ..
 #pragma unroll
-  for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-    for (int ob = 0; ob < 4; ++ob) w2t[ib][ob] = lds4(&img->w2tf[((ib * 4 + ob) * 64 + l) * 4]);
+  for (int ob = 0; ob < 4; ++ob) w2t[ob] = lds4(&img->w2tf[((w * 4 + ob) * 64 + l) * 4]);
 
-  f32x4 gW1[4][2], gW2[4][4];
+  f32x4 gW1[2], gW2[4];
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
+  for (int b = 0; b < 2; ++b) gW1[b] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int b = 0; b < 2; ++b) gW1[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < 4; ++b) gW2[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float gb1[4], gb2[4], gw3[4];  // per lane: hidden 16 w + 4 g + r
 #pragma unroll
-    for (int b = 0; b < 4; ++b) gW2[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  float gb1[16], gb2[16], gw3[16];  // per lane: hidden blk*16 + 4g + r (blk = idx / 4, r = idx % 4)
-#pragma unroll
-  for (int i = 0; i < 16; ++i) gb1[i] = gb2[i] = gw3[i] = 0.f;
+  for (int r = 0; r < 4; ++r) gb1[r] = gb2[r] = gw3[r] = 0.f;
   float gb3 = 0.f, loss = 0.f;
 
-  for (int tile = gw; tile < ntiles; tile += nw) {
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     Tile t;
     load_tile(x, n, tile, t);
     const int e = tile * 16 + c;
@@ -128,107 +124,88 @@ __global__ __launch_bounds__(64) void mlp_grad_kernel(const TrainImage *__restri
     }
     const float dout = 2.f * res * t.y * (1.f - t.y) * inv_n;  // dL/do for element c
     // layer 3 and layer 2 backward (C layout)
-    f32x4 d2[4];
+    bf16x4 d2b[4], d2w = {0, 0, 0, 0};
 #pragma unroll
     for (int ob = 0; ob < 4; ++ob) {
+      float d2[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float z = t.z2[ob][r];
-        gw3[ob * 4 + r] += dout * (z > 0.f ? z : 0.f);
-        const float dz = z > 0.f ? wr.w3[ob][r] * dout : 0.f;
-        d2[ob][r] = dz;
-        gb2[ob * 4 + r] += dz;
+      for (int r = 0; r < 4; ++r) d2[r] = t.z2[ob][r] > 0.f ? wr.w3[ob][r] * dout : 0.f;
+      d2b[ob] = pack4(d2[0], d2[1], d2[2], d2[3]);
+      if (ob == w) {
+        d2w = d2b[ob];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float z = t.z2[ob][r];
+          gw3[r] += dout * (z > 0.f ? z : 0.f);
+          gb2[r] += d2[r];
+        }
       }
     }
-    bf16x4 d2b[4];
+    // rows 16 w .. of dH1^T = W2^T dZ2^T, then through the first ReLU
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, z1 = t.z1[0];
 #pragma unroll
-    for (int ob = 0; ob < 4; ++ob) d2b[ob] = pack4(d2[ob][0], d2[ob][1], d2[ob][2], d2[ob][3]);
-    // dH1^T = W2^T dZ2^T, then through the first ReLU
-    f32x4 d1[4];
+    for (int ob = 0; ob < 4; ++ob) acc = mfma(w2t[ob], d2b[ob], acc);
 #pragma unroll
-    for (int ib = 0; ib < 4; ++ib) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int b = 1; b < 4; ++b)
+      if (b == w) z1 = t.z1[b];
+    float d1[4];
 #pragma unroll
-      for (int ob = 0; ob < 4; ++ob) acc = mfma(w2t[ib][ob], d2b[ob], acc);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float dz = t.z1[ib][r] > 0.f ? acc[r] : 0.f;
-        d1[ib][r] = dz;
-        gb1[ib * 4 + r] += dz;
-      }
+    for (int r = 0; r < 4; ++r) {
+      d1[r] = z1[r] > 0.f ? acc[r] : 0.f;
+      gb1[r] += d1[r];
     }
     // transposes: [hidden][element] images of X, H1, dZ2, dZ1 (BF16)
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s_x[(kb * 16 + 4 * g + j) * 16 + c] = (uint16_t)t.xb[kb][j];
+      for (int j = 0; j < 4; ++j) s_x[w][(kb * 16 + 4 * g + j) * 16 + c] = (uint16_t)t.xb[kb][j];
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int row = (b * 16 + 4 * g + j) * 16 + c;
-        s_h1[row] = (uint16_t)t.h1b[b][j];
-        s_d2[row] = (uint16_t)d2b[b][j];
-        s_d1[row] = to_bf16(d1[b][j]);
-      }
+      for (int j = 0; j < 4; ++j) s_h1[w][(b * 16 + 4 * g + j) * 16 + c] = (uint16_t)t.h1b[b][j];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      s_d2[w][(4 * g + j) * 16 + c] = (uint16_t)d2w[j];
+      s_d1[w][(4 * g + j) * 16 + c] = to_bf16(d1[j]);
+    }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     // dW2 (out x in) += dZ2^T H1: A = dZ2^T rows, B = H1 columns, K = element
+    const bf16x4 a2 = lds4(&s_d2[w][c * 16 + 4 * g]);
 #pragma unroll
-    for (int ob = 0; ob < 4; ++ob) {
-      const bf16x4 a = lds4(&s_d2[(ob * 16 + c) * 16 + 4 * g]);
-#pragma unroll
-      for (int ib = 0; ib < 4; ++ib) gW2[ob][ib] = mfma(a, lds4(&s_h1[(ib * 16 + c) * 16 + 4 * g]), gW2[ob][ib]);
-    }
+    for (int ib = 0; ib < 4; ++ib) gW2[ib] = mfma(a2, lds4(&s_h1[w][(ib * 16 + c) * 16 + 4 * g]), gW2[ib]);
     // dW1 (hidden x feature) += dZ1^T X
+    const bf16x4 a1 = lds4(&s_d1[w][c * 16 + 4 * g]);
 #pragma unroll
-    for (int hb = 0; hb < 4; ++hb) {
-      const bf16x4 a = lds4(&s_d1[(hb * 16 + c) * 16 + 4 * g]);
-#pragma unroll
-      for (int fb = 0; fb < 2; ++fb) gW1[hb][fb] = mfma(a, lds4(&s_x[(fb * 16 + c) * 16 + 4 * g]), gW1[hb][fb]);
-    }
+    for (int fb = 0; fb < 2; ++fb) gW1[fb] = mfma(a1, lds4(&s_x[w][(fb * 16 + c) * 16 + 4 * g]), gW1[fb]);
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   }
 
-  // per-lane vectors summed over the 16 lanes of a row group (elements)
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    gb1[i] = row_sum(gb1[i]);
-    gb2[i] = row_sum(gb2[i]);
-    gw3[i] = row_sum(gw3[i]);
-  }
-  gb3 = row_sum(gb3);
-  loss = row_sum(loss);
-  float *row = partial + (size_t)gw * NPL;
+  float *row = partial + (size_t)blockIdx.x * NPL;
   // accumulator layout: row 4g + r, column c of each 16 x 16 tile
 #pragma unroll
-  for (int hb = 0; hb < 4; ++hb)
+  for (int r = 0; r < 4; ++r) {
+    const int h = w * 16 + 4 * g + r;
 #pragma unroll
     for (int fb = 0; fb < 2; ++fb)
+      if (fb * 16 + c < NF) row[OFF_W1 + h * NF + fb * 16 + c] = gW1[fb][r];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int h = hb * 16 + 4 * g + r, f = fb * 16 + c;
-        if (f < NF) row[OFF_W1 + h * NF + f] = gW1[hb][fb][r];
-      }
-#pragma unroll
-  for (int ob = 0; ob < 4; ++ob)
-#pragma unroll
-    for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) row[OFF_W2 + (ob * 16 + 4 * g + r) * NH + ib * 16 + c] = gW2[ob][ib][r];
-  if (c == 0) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int h = (i / 4) * 16 + 4 * g + (i % 4);
-      row[OFF_B1 + h] = gb1[i];
-      row[OFF_B2 + h] = gb2[i];
-      row[OFF_W3 + h] = gw3[i];
+    for (int ib = 0; ib < 4; ++ib) row[OFF_W2 + h * NH + ib * 16 + c] = gW2[ib][r];
+    // per-lane vectors summed over the 16 lanes of a row group (elements)
+    const float s1 = row_sum(gb1[r]), s2 = row_sum(gb2[r]), s3 = row_sum(gw3[r]);
+    if (c == 0) {
+      row[OFF_B1 + h] = s1;
+      row[OFF_B2 + h] = s2;
+      row[OFF_W3 + h] = s3;
     }
   }
-  if (l == 0) {
-    row[OFF_B3] = gb3;
-    row[NP] = loss;
+  if (w == 0) {
+    const float s = row_sum(gb3), ls = row_sum(loss);
+    if (l == 0) {
+      row[OFF_B3] = s;
+      row[NP] = ls;
+    }
   }
 }
 
@@ -244,7 +221,8 @@ __global__ __launch_bounds__(64) void mlp_grad_kernel(const TrainImage *__restri
 // weights w with the moments m and v, and the new weight into the images, by the
 // thread that holds the gradient's sum. As four launches (reduction with two
 // loads in flight, Adam, packing by one workgroup) a training step on 8192
-// elements took 58 us, with this 24.
+// elements took 58 us, with this and 256 rows 20
+// us (the reduction alone 19.9 and 4.2 us).
 constexpr int RED_COLS = 32, RED_SPLIT = 8, RED_BATCH = 32;
 struct AdamArgs {
   float *w, *m, *v;

@@ -98,7 +98,11 @@ constexpr int kMaxPartials = 1 << 16;
 constexpr int kMaxSpeedBlocks = 1 << 16;  // workgroups (and partials) of the wave-speed reduction
 constexpr int kAnalysisBlocks = 1024;  // workgroups of the error norms; twice as many of the integrals
 static_assert(2 * kAnalysisBlocks * 10 <= kMaxPartials, "their partial results fit");
-constexpr int kMlpMaxWaves = 1024;  // partial gradient rows of one training step
+// partial gradient rows of one training step: one workgroup for each CU. Rows of 22 KB
+// are written and read again, more of them cost more than a second tile for a workgroup
+// (20 Adam steps with 256 against 1024 rows: 19.8 and 23.8 us each on 8192 elements,
+// 24.1 and 34.3 us on 20000, 40.4 and 42.9 us on 65536; 128 rows: 19.8, 28.7, 61.2 us)
+constexpr int kMlpMaxRows = 256;
 constexpr int kEagerSolveSteps = 8;  // trixi_hip_solve with at most this many steps launches without graphs
 
 }  // namespace
@@ -518,9 +522,9 @@ int launch_hg(trixi_hip_ctx *ctx, const S *u, double *alpha_out, float *feat, co
   return TRIXI_HIP_OK;
 }
 
-// wavefronts of a launch over n elements (16 to a tile)
-int mlp_waves(int n) { return std::min(std::max((n + 15) / 16, 1), kMlpMaxWaves); }
-int mlp_blocks(int n) { return (mlp_waves(n) + mlp::WAVES - 1) / mlp::WAVES; }
+// tiles of 16 elements that a launch over n elements works on at a time
+int mlp_tiles(int n) { return std::min(std::max((n + 15) / 16, 1), kMlpMaxRows); }
+int mlp_blocks(int n) { return (mlp_tiles(n) + mlp::WAVES - 1) / mlp::WAVES; }
 
 // Raw (unsmoothed) blending factors of state u into alpha_out, from the
 // indicator selected by ind_mode.
@@ -1643,7 +1647,7 @@ static int mlp_check(trixi_hip_ctx *ctx) {
   HIP_TRY(dev_alloc(ctx, &ctx->d_mlp, nmlp * 4));
   HIP_TRY(dev_alloc(ctx, &ctx->d_feat, (size_t)ctx->E * kMlpFeatureStride * 4));
   HIP_TRY(dev_alloc(ctx, &ctx->d_alpha_hg, (size_t)ctx->E * 8));
-  HIP_TRY(dev_alloc(ctx, &ctx->d_mlp_partial, (size_t)kMlpMaxWaves * mlp::NPL * 4));
+  HIP_TRY(dev_alloc(ctx, &ctx->d_mlp_partial, (size_t)kMlpMaxRows * mlp::NPL * 4));
   HIP_TRY(dev_alloc(ctx, &ctx->d_mlp_img, sizeof(mlp::TrainImage)));
   return TRIXI_HIP_OK;
 }
@@ -1729,8 +1733,8 @@ int trixi_hip_mlp_forward(trixi_hip_ctx *ctx, const float *x_dev, int n, float *
 // Gradient and loss into the gradient buffer; with adam also the training step.
 static int mlp_gradient(trixi_hip_ctx *ctx, const float *x_dev, const float *target_dev, int n,
                         const mlp::AdamArgs *adam) {
-  const int rows = mlp_waves(n);
-  hipLaunchKernelGGL(mlp::mlp_grad_kernel, dim3(rows), dim3(64), 0, ctx->stream, ctx->d_mlp_img, x_dev, target_dev, n,
+  const int rows = mlp_tiles(n);
+  hipLaunchKernelGGL(mlp::mlp_grad_kernel, dim3(rows), dim3(256), 0, ctx->stream, ctx->d_mlp_img, x_dev, target_dev, n,
                      ctx->d_mlp_partial);
   HIP_TRY(hipGetLastError());
   hipLaunchKernelGGL(adam ? mlp::mlp_reduce_kernel<true> : mlp::mlp_reduce_kernel<false>,
