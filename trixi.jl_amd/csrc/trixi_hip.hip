@@ -186,10 +186,11 @@ struct trixi_hip_ctx {
   int xcd_remap = 1;
   // the last stage of a step reduces the wave speed in its epilogue (see
   // stage_wave_speed) instead of max_speed_nodes_kernel reading the state again.
-  // FP32 default: 3D p3 CK2N54 step 382.6 -> 370.4 us. FP64 is slower with it
-  // (611.6 vs 623.2 us: at two workgroups per CU the epilogue's barriers are not
-  // hidden). A/B on one box; TRIXI_HIP_FUSED_SPEED=0/1 overrides.
-  bool fused_speed = false;
+  // FP32 3D p3 CK2N54 step 382.6 -> 370.4 us. FP64: 128^2 elements p3 with shock
+  // capturing 112 -> 100 us, 3D p3 on 16^3 elements 105 -> 102 us, on 32^3 619 -> 618
+  // us; 2D and 3D p2 to p4 on 8 to 65 536 elements 0.998 to 1.115 times as fast. A/B
+  // on one box; TRIXI_HIP_FUSED_SPEED=0 turns it off.
+  bool fused_speed = true;
 
   // captured RK steps, keyed by scheme, stream, entry point and start parity
   // (two slots: consecutive steps of a scheme with an odd stage count alternate)
@@ -1001,7 +1002,6 @@ int trixi_hip_create(const trixi_hip_config *cfg, const trixi_hip_mesh *mesh,
   ctx->hg.threshold = 0.5 * std::pow(10.0, -1.8 * std::pow((double)n, 0.25));
   ctx->hg.parameter_s = std::log((1 - 0.0001) / 0.0001);
   ctx->hg.variable = cfg->hg_variable;
-  ctx->fused_speed = cfg->precision == TRIXI_HIP_FP32;
   if (const char *env = std::getenv("TRIXI_HIP_FUSED_INDICATOR")) ctx->fused_ind = std::atoi(env) != 0;
   if (const char *env = std::getenv("TRIXI_HIP_XCD_REMAP")) ctx->xcd_remap = std::atoi(env) != 0;
   if (const char *env = std::getenv("TRIXI_HIP_FUSED_SPEED")) ctx->fused_speed = std::atoi(env) != 0;
