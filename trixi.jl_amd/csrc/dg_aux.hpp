@@ -493,10 +493,10 @@ template <int D, int N> struct NormsTile {
 // LDS, the others in registers, each thread owning one column of analysis nodes
 // along the last. The coordinates vary along their own dimension only. Sums stay in
 // registers over a workgroup's tiles, so that one reduction of 2 V values follows
-// a launch's ~1000 workgroups. 123 us for 3D p3 on 32^3 elements; an analysis, with
-// the integrals below, takes 194 us. With the product over all (N + 1)^D nodes for each
-// analysis node, one workgroup and reduction for each element, and its 32 768 rows
-// summed by one workgroup, it took 2 084 us.
+// a launch's ~1000 workgroups. 109 us for 3D p3 on 32^3 elements (123 us with a
+// loop over the tile's loads, a memory round trip each); 1 674 us with the product
+// over all (N + 1)^D nodes for each analysis node and one workgroup and reduction
+// for each element.
 template <int D, int N, bool PLAIN>
 __global__ __launch_bounds__(256, PLAIN && N < 4 ? 3 : 1) void error_norms_kernel(const double *__restrict__ u,
                                                           const double *__restrict__ inv_jac,
@@ -523,8 +523,17 @@ __global__ __launch_bounds__(256, PLAIN && N < 4 ? 3 : 1) void error_norms_kerne
   const int a0 = col % NA, a1 = D == 3 ? col / NA : 0;
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const int e0 = tile * EB, ne = min(EB, E - e0);
+    // all loads of the tile's state in flight at once (in bounds also past its end)
+    constexpr int RPT = (EB * NN * V + 255) / 256;
+    const int nv = ne * NN * V;
+    double r[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) r[k] = u[(size_t)e0 * NN * V + min(tid + k * 256, nv - 1)];
+    const double ij = inv_jac[e0 + min(el_c, ne - 1)];
     __syncthreads();  // the previous tile is consumed; s_vdm is complete
-    for (int i = tid; i < ne * NN * V; i += 256) s_u[i] = u[(size_t)e0 * NN * V + i];
+#pragma unroll
+    for (int k = 0; k < RPT; ++k)
+      if (tid + k * 256 < nv) s_u[tid + k * 256] = r[k];
     for (int i = tid; i < ne * D * NA; i += 256) {
       const int a = i % NA, ed = i / NA, el = ed / D, d = ed - el * D;
       const double jac = 1.0 / inv_jac[e0 + el], c = centers[d + D * (e0 + el)];
@@ -565,7 +574,7 @@ __global__ __launch_bounds__(256, PLAIN && N < 4 ? 3 : 1) void error_norms_kerne
           }
           val[k][v] = y;
         }
-      const double jac = 1.0 / inv_jac[e0 + el_c];
+      const double jac = 1.0 / ij;
       const double vol = D == 3 ? jac * jac * jac : jac * jac;
       const double wc = D == 3 ? ac.aw[a0] * ac.aw[a1] : ac.aw[a0];
       double x[D];
@@ -598,8 +607,9 @@ __global__ __launch_bounds__(256, PLAIN && N < 4 ? 3 : 1) void error_norms_kerne
 // integrate_via_indices (analysis_dg3d.jl:364-386) of u and entropy_math
 // (compressible_euler_3d.jl:1970-1976): partial[workgroup] = {int u [V], int S}.
 // One thread per node, walking the nodes at the stride of the launch, so that a
-// wavefront reads 2.5 KB in one piece (one thread per element read at that stride):
-// bound by the read of the state, 23 us for 84 MB (3D p3 on 32^3 elements).
+// wavefront reads 2.5 KB in one piece: bound by the read of the state, 23 us for 84
+// MB (3D p3 on 32^3 elements). One thread per element, reading at a stride of 2.5
+// KB, took 46 us.
 template <int D, int N>
 __global__ __launch_bounds__(256) void integrals_kernel(const double *__restrict__ u,
                                                         const double *__restrict__ inv_jac,
@@ -639,8 +649,9 @@ __global__ __launch_bounds__(256) void integrals_kernel(const double *__restrict
 }
 
 // Column blockIdx.x of a partial table [rows, cols] -> out: its sum, or its
-// maximum (NaN wins) for columns from nsum on. One workgroup for each column: 5 us;
-// one workgroup for all of them took 34 us for 10 columns of 6000 rows.
+// maximum (NaN wins) for columns from nsum on. One workgroup for each column: 5 us
+// for 937 rows of 10 columns or 2048 of 6. One workgroup for all columns, a row for each
+// of 32 768 elements: 216 and 118 us.
 static __global__ __launch_bounds__(256) void reduce_columns_kernel(const double *__restrict__ partial, int rows,
                                                                     int cols, int nsum, double *__restrict__ out) {
   __shared__ double s_red[4];
