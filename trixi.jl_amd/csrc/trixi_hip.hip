@@ -96,8 +96,8 @@ template <typename F> bool dispatch_dn(int D, int N, F &&f) {
 
 constexpr int kMaxPartials = 1 << 16;
 constexpr int kMaxSpeedBlocks = 1 << 16;  // workgroups (and partials) of the wave-speed reduction
-constexpr int kAnalysisBlocks = 1024;  // workgroups of the error norms; twice as many of the integrals
-static_assert(2 * kAnalysisBlocks * 10 <= kMaxPartials, "their partial results fit");
+constexpr int kIntegralBlocks = 2048;  // workgroups of the integrals; the error norms have at most 768
+static_assert(kIntegralBlocks * 6 <= kMaxPartials && 768 * 10 <= kMaxPartials, "their partial results fit");
 // partial gradient rows of one training step: one workgroup for each CU. Rows of 22 KB
 // are written and read again, more of them cost more than a second tile for a workgroup
 // (20 Adam steps with 256 against 1024 rows: 19.8 and 23.8 us each on 8192 elements,
@@ -1317,9 +1317,11 @@ int enqueue_error_sums(trixi_hip_ctx *ctx, double t, const double *tdev, double 
     for (int i = 0; i < NA * (N + 1); ++i) ac.vdm[i] = ctx->a_vdm[i];
     for (int i = 0; i < NA; ++i) ac.aw[i] = ctx->a_weights[i];
     for (int i = 0; i <= N; ++i) ac.nodes[i] = ctx->nodes[i];
-    // as many tiles for each of up to kAnalysisBlocks workgroups (3 or 4 fit a CU)
+    // as many tiles for each of the workgroups that run at once, or of half of them
+    // where one fits a CU: with 937 workgroups for 768 places the last 169 ran alone
     const int tiles = (E + NormsTile<D, N>::EB - 1) / NormsTile<D, N>::EB;
-    const int each = (tiles + kAnalysisBlocks - 1) / kAnalysisBlocks;
+    const int most = 256 * (plain_exact(ctx->exact) && N < 4 ? 3 : 2);
+    const int each = (tiles + most - 1) / most;
     blocks = (tiles + each - 1) / each;
     hipLaunchKernelGGL((plain_exact(ctx->exact) ? error_norms_kernel<D, N, true> : error_norms_kernel<D, N, false>),
                        dim3(blocks), dim3(256), 0, ctx->stream, cur_u64(ctx), ctx->d_invj, ctx->d_centers, E, t, tdev,
@@ -1336,7 +1338,7 @@ int enqueue_error_sums(trixi_hip_ctx *ctx, double t, const double *tdev, double 
 // integrate_via_indices sums of u and the mathematical entropy -> out[0, V + 1).
 int enqueue_integral_sums(trixi_hip_ctx *ctx, double *out) {
   const int V = ctx->V, E = ctx->E;
-  const int blocks = (int)std::min<size_t>(((size_t)E * ctx->NN + 255) / 256, 2 * kAnalysisBlocks);
+  const int blocks = (int)std::min<size_t>(((size_t)E * ctx->NN + 255) / 256, kIntegralBlocks);
   bool ok = dispatch_dn(ctx->D, ctx->N, [&](auto Dc, auto Nc) {
     constexpr int D = decltype(Dc)::value, N = decltype(Nc)::value;
     hipLaunchKernelGGL((integrals_kernel<D, N>), dim3(blocks), dim3(256), 0, ctx->stream, cur_u64(ctx), ctx->d_invj, E,
