@@ -573,8 +573,10 @@ int launch_before_element(trixi_hip_ctx *ctx, const S *u, double t, const double
   // outer states of the Dirichlet boundaries at this stage's time; a
   // time-independent boundary function is evaluated once
   const bool t_dep = ctx->exact.kind == TRIXI_HIP_IC_CONVERGENCE_TEST;
-  if (ctx->B > 0 && !ctx->slip && (t_dep || !ctx->ghost_ready)) {
-    ctx->ghost_ready = !t_dep;
+  const bool states = ctx->B > 0 && !ctx->slip && (t_dep || !ctx->ghost_ready);
+  const bool with_mortars = states && t_dep && ctx->M > 0;  // the mortars' launch evaluates them
+  if (states) ctx->ghost_ready = !t_dep;
+  if (states && !with_mortars) {
     bool ok = dispatch_dn(ctx->D, ctx->N, [&](auto Dc, auto Nc) {
       constexpr int D = decltype(Dc)::value, N = decltype(Nc)::value;
       const int total = ctx->B * ipow_c(N + 1, D - 1);
@@ -605,9 +607,11 @@ int launch_before_element(trixi_hip_ctx *ctx, const S *u, double t, const double
         mc.ru[i] = T(ctx->mru[i]);
         mc.rl[i] = T(ctx->mrl[i]);
       }
-      hipLaunchKernelGGL((mortar_flux_kernel<T, D, N, S>), dim3((ctx->M + MPB - 1) / MPB), dim3(256), 0, ctx->stream,
-                         u, ctx->d_mort, ctx->M, ctx->B, ctx->cfg.surface_flux, T(ctx->cfg.gamma), mc,
-                         (T *)ctx->d_mflux);
+      const int mblocks = (ctx->M + MPB - 1) / MPB;
+      const int bnodes = with_mortars ? ctx->B * ipow_c(n, D - 1) : 0;
+      hipLaunchKernelGGL((mortar_flux_kernel<T, D, N, S>), dim3(mblocks + (bnodes + 255) / 256), dim3(256), 0,
+                         ctx->stream, u, ctx->d_mort, ctx->M, ctx->B, ctx->cfg.surface_flux, T(ctx->cfg.gamma), mc,
+                         (T *)ctx->d_mflux, mblocks, ctx->d_bx, bnodes, t, tdev, (T *)ctx->d_ghost);
     });
     if (!ok) return TRIXI_HIP_EINVAL;
     HIP_TRY(hipGetLastError());
