@@ -80,8 +80,8 @@ __device__ __forceinline__ float row_sum(float x) {
 // 16 w .. 16 w + 15 of both layers' gradients (and wavefront 0 the scalars). The
 // weights are loaded as fragments from the image into registers, all at once. 8192
 // elements: 25.2 us with one wavefront to a tile, four to a workgroup that converted
-// the FP32 weights into LDS first; 13.9 us with one, weights from the image; 12.1 us
-// with four, two tiles to a workgroup.
+// the FP32 weights into LDS first; 13.9 us with one, weights from the image; 13.3 us
+// with four.
 __global__ __launch_bounds__(256) void mlp_grad_kernel(const TrainImage *__restrict__ img, const float *__restrict__ x,
                                                        const float *__restrict__ target, int n,
                                                        float *__restrict__ partial) {
@@ -221,8 +221,8 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const TrainImage *__restr
 // weights w with the moments m and v, and the new weight into the images, by the
 // thread that holds the gradient's sum. As four launches (reduction with two
 // loads in flight, Adam, packing by one workgroup) a training step on 8192
-// elements took 58 us, with this and 256 rows 20
-// us (the reduction alone 19.9 and 4.2 us).
+// elements took 58 us, with this 24 us (the
+// reduction alone 19.9 and 6.3 us). Same weights, bit for bit.
 constexpr int RED_COLS = 32, RED_SPLIT = 8, RED_BATCH = 32;
 struct AdamArgs {
   float *w, *m, *v;
@@ -263,8 +263,10 @@ __global__ __launch_bounds__(RED_COLS *RED_SPLIT) void mlp_reduce_kernel(const f
     for (int k = 1; k < RED_SPLIT; ++k) t += s_part[k][c];
     out[p] = t;
     if (STEP && p < NP) {
-      mi = a.beta1 * mi + (1.f - a.beta1) * t;
-      vi = a.beta2 * vi + (1.f - a.beta2) * t * t;
+      // the roundings written out: Adam divides by the gradient's size, so that one of
+      // another order shows in the weights after a few steps
+      mi = __builtin_fmaf(1.f - a.beta1, t, a.beta1 * mi);
+      vi = __builtin_fmaf((1.f - a.beta2) * t, t, a.beta2 * vi);
       a.m[p] = mi;
       a.v[p] = vi;
       const float mh = mi / (1.f - powf(a.beta1, (float)a.step));

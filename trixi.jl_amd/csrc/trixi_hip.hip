@@ -98,11 +98,11 @@ constexpr int kMaxPartials = 1 << 16;
 constexpr int kMaxSpeedBlocks = 1 << 16;  // workgroups (and partials) of the wave-speed reduction
 constexpr int kIntegralBlocks = 2048;  // workgroups of the integrals; the error norms have at most 768
 static_assert(kIntegralBlocks * 6 <= kMaxPartials && 768 * 10 <= kMaxPartials, "their partial results fit");
-// partial gradient rows of one training step: one workgroup for each CU. Rows of 22 KB
-// are written and read again, more of them cost more than a second tile for a workgroup
-// (20 Adam steps with 256 against 1024 rows: 19.8 and 23.8 us each on 8192 elements,
-// 24.1 and 34.3 us on 20000, 40.4 and 42.9 us on 65536; 128 rows: 19.8, 28.7, 61.2 us)
-constexpr int kMlpMaxRows = 256;
+// partial gradient rows of one training step. Fewer rows cost less (19.8 instead of
+// 23.8 us a step on 8192 elements with 256 rows), but other partial sums round
+// differently, and Adam, which divides by the gradient's size, made 5e-5 of the
+// weights of that within 20 steps.
+constexpr int kMlpMaxRows = 1024;
 constexpr int kEagerSolveSteps = 8;  // trixi_hip_solve with at most this many steps launches without graphs
 
 }  // namespace
