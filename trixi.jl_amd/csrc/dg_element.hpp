@@ -411,14 +411,21 @@ __device__ __forceinline__ void line_faces(const ElemArgs<T> &a, const DGConst<T
           }
         }
       };
+      // The neighbour's sound speed. In FP64 in the same operations as the records',
+      // sqrt(gamma) sqrt(p / rho): the element on the other side swaps the two
+      // states, and both have to find the same flux.
+      auto sound = [&](const ConsP<T, D> &x) {
+        if constexpr (F64) return a.sqrt_gamma * Prec<T>::sqrt_(x.p * x.irho);
+        else return Prec<T>::sqrt_(gamma * x.p * x.irho);
+      };
       ConsP<T, D> nb;
       consp_from_cons<T, D>(c.ul_m, gm1, nb);  // -O face: element is the right state
-      flux_llf_pc2<T, D, O>(nb, own_face[0], Prec<T>::sqrt_(gamma * nb.p * nb.irho), own_c[0], naive, F);
+      flux_llf_pc2<T, D, O>(nb, own_face[0], sound(nb), own_c[0], naive, F);
       given_flux2(c.fm, F);
 #pragma unroll
       for (int v = 0; v < V; ++v) acc[0][v] = tfma(-F[v], hfactor, acc[0][v]);
       consp_from_cons<T, D>(c.ur_p, gm1, nb);  // +O face: element is the left state
-      flux_llf_pc2<T, D, O>(own_face[1], nb, own_c[1], Prec<T>::sqrt_(gamma * nb.p * nb.irho), naive, F);
+      flux_llf_pc2<T, D, O>(own_face[1], nb, own_c[1], sound(nb), naive, F);
       given_flux2(c.fp, F);
 #pragma unroll
       for (int v = 0; v < V; ++v) acc[n - 1][v] = tfma(F[v], hfactor, acc[n - 1][v]);
