@@ -16,6 +16,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "log_mean.hpp"
+
 namespace trixi_hip {
 
 enum VolumeKind { VOL_WEAK = 0, VOL_FD_RANOCHA = 1, VOL_FD_CENTRAL = 2, VOL_HG_RANOCHA = 3,
@@ -265,7 +267,7 @@ __device__ __forceinline__ void flux_ranocha_fast(const NodeR<float, D> &l, cons
 // Per-node data of the FP64 flux_ranocha lines: the roots r of the density and
 // t of the temperature T = p/rho (1/T is the beta of the means above, and
 // sqrt(gamma) t the sound speed), half velocities, half pressure. No logarithms
-// are stored: two per node cost more than the series of means_near, and the
+// are stored: two per node cost more than the series of log_means, and the
 // line's records take fewer registers (three wavefronts per SIMD for polydeg 3
 // and 4 in 3D).
 template <int D> struct NodeD {
@@ -306,91 +308,14 @@ __device__ __forceinline__ void flux_ranocha_tail(const NodeD<D> &l, const NodeD
   f[D + 1] = tfma(f1, tfma(inv_rho_p_mean, half_inv_gamma_m1, hh), cross);
 }
 
-// Logarithmic means without logarithms. With a = sqrt(x), b = sqrt(y) and f = (b -
-// a) / (b + a), ln(y/x) = 4 atanh f and y - x = 4 a b f / (1 - f^2), so
-//   ln_mean(x, y)     = a b S(f^2), S = f / ((1 - f^2) atanh f),
-//   x y / ln_mean(x, y) = a b R(f^2), R = 1 / S,
-// products of the roots with functions near 1, replaced by their Chebyshev
-// interpolants on f^2 in [0, fmax^2]: for roots within a factor 23/17 (|f| <= 0.15,
-// values within 1.83) of degrees 7 and 6 (relative error 9.7e-19 and 4.0e-18), for roots
-// within a factor 2 (|f| <= 1/3, values within 4) of degrees 10 and 9 (1.2e-17 and
-// 5.3e-18).
-struct MeanSeriesShort {
-  static constexpr uint32_t kMaxSpread = 370084;  // (23/17 - 1) 2^20, less one for the low words
-  static constexpr double s[] = {1.0, 0.6666666666666721, 0.5777777777726917, 0.5312169330222599,
-      0.5010226133709935, 0.47925578566700217, 0.4608934367742883, 0.4904778843261837};
-  static constexpr double r[] = {1.0, -0.6666666666666498, -0.1333333333453491, -0.057142853944403244,
-      -0.03174643661749843, -0.020175779003228016, -0.014824140918770774};
-};
-struct MeanSeriesLong {
-  static constexpr uint32_t kMaxSpread = 1048575;  // (2 - 1) 2^20, less one for the low words
-  static constexpr double s[] = {1.0, 0.6666666666666411, 0.5777777777869698, 0.5312169299318927,
-      0.5010230195983105, 0.47922230088317014, 0.46253726376812154, 0.44731039085063473, 0.45473529811358404,
-      0.3202068928099197, 0.786358922620139};
-  static constexpr double r[] = {1.0, -0.6666666666666746, -0.133333333330976, -0.05714285741322125,
-      -0.031746016040014965, -0.020202542412086334, -0.013975499645365397, -0.010386267724833162,
-      -0.006890815785775918, -0.009891136741349926};
-};
-__device__ __forceinline__ uint32_t high_word(double x) {
-  return (uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32);
-}
-template <int N> __device__ __forceinline__ double horner(const double (&c)[N], double z) {
-  double a = c[N - 1];
-#pragma unroll
-  for (int k = N - 2; k >= 0; --k) a = tfma(a, z, c[k]);
-  return a;
-}
-// c ? a : b with both values computed: as a plain conditional the compiler makes
-// a branch of it and, pair after pair, a control flow that keeps all values live.
-__device__ __forceinline__ double select(bool c, double a, double b) {
-  asm volatile("" : "+v"(a), "+v"(b));
-  return c ? a : b;
-}
-// The form of a line's means: short or long series, or logarithms.
-enum MeanKind { MEAN_SHORT = 0, MEAN_LONG = 1, MEAN_LOG = 2 };
-// Means of the series: ln_mean of the densities, and 1/ln_mean(1/T_l, 1/T_r) = T_l
-// T_r / ln_mean(T_l, T_r). MIXED selects the series by kind (of the lane's line),
-// else it is the short one. One reciprocal serves both sums, 1/s1 = s2 / (s1 s2)
-// and 1/s2 = s1 / (s1 s2).
-template <bool MIXED, int D>
-__device__ __forceinline__ void means_near(const NodeD<D> &l, const NodeD<D> &r, int kind, double &rho_mean,
-                                           double &inv_rho_p_mean) {
-  using A = MeanSeriesShort;
-  using B = MeanSeriesLong;
-  const double s1 = l.r + r.r, d1 = r.r - l.r, s2 = l.t + r.t, d2 = r.t - l.t;
-  const double is = Prec<double>::rcp(s1 * s2);
-  const double f1 = d1 * (is * s2), f2 = d2 * (is * s1);
-  const double z1 = f1 * f1, z2 = f2 * f2;
-  double ps = horner(A::s, z1), pr = horner(A::r, z2);
-  if constexpr (MIXED) {
-    ps = select(kind == MEAN_SHORT, ps, horner(B::s, z1));
-    pr = select(kind == MEAN_SHORT, pr, horner(B::r, z2));
-  }
-  rho_mean = (l.r * r.r) * ps;
-  inv_rho_p_mean = (l.t * r.t) * pr;
-}
-// FP64 flux_ranocha without logarithms. As in the FP32 variant the energy
-// component is returned halved.
-template <bool MIXED, int D, int O>
-__device__ __forceinline__ void flux_ranocha_near(const NodeD<D> &l, const NodeD<D> &r, int kind,
-                                                  double half_inv_gamma_m1, double *f) {
+// FP64 flux_ranocha of two node records (log_means). As in the FP32 variant the
+// energy component is returned halved.
+template <bool LOGS, bool ORDERED, int D, int O>
+__device__ __forceinline__ void flux_ranocha_d(const NodeD<D> &l, const NodeD<D> &r, double ln_rho, double ln_t,
+                                               double half_inv_gamma_m1, double *f) {
   double rho_mean, inv_rho_p_mean;
-  means_near<MIXED, D>(l, r, kind, rho_mean, inv_rho_p_mean);
-  flux_ranocha_tail<D, O>(l, r, rho_mean, inv_rho_p_mean, half_inv_gamma_m1, f);
-}
-
-// The same where some line of the wavefront needs logarithms (of the roots).
-template <int D, int O>
-__device__ __forceinline__ void flux_ranocha_far(const NodeD<D> &l, const NodeD<D> &r, int kind, double lr_l,
-                                                 double lr_r, double lt_l, double lt_r, double half_inv_gamma_m1,
-                                                 double *f) {
-  double rho_mean, inv_rho_p_mean;
-  means_near<true, D>(l, r, kind, rho_mean, inv_rho_p_mean);
-  const double tl = l.t * l.t, tr = r.t * r.t;
-  const double rho_log = ln_mean_l(l.r * l.r, r.r * r.r, 2 * lr_l, 2 * lr_r);
-  const double inv_log = (tl * tr) * inv_ln_mean_l(tl, tr, 2 * lt_l, 2 * lt_r);
-  rho_mean = select(kind == MEAN_LOG, rho_log, rho_mean);
-  inv_rho_p_mean = select(kind == MEAN_LOG, inv_log, inv_rho_p_mean);
+  log_means<LOGS, ORDERED>(l.r, r.r, l.t, r.t, ln_rho, ln_t, [](double x) { return Prec<double>::rcp(x); }, rho_mean,
+                           inv_rho_p_mean);
   flux_ranocha_tail<D, O>(l, r, rho_mean, inv_rho_p_mean, half_inv_gamma_m1, f);
 }
 

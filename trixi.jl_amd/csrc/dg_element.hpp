@@ -444,15 +444,35 @@ __device__ __forceinline__ void line_faces(const ElemArgs<T> &a, const DGConst<T
   }
 }
 
+// Whether an FP64 flux_ranocha line may hold a pair outside the range of the
+// means' series. The high words h of two positive doubles order them, and their
+// quotient is at most 1 + (h1 - h0) 2^-20 while that is below 2 (the high word grows
+// linearly within a binade, so per factor slowest at its start). So the largest minus
+// the smallest high word of the line's roots bounds every pair's |f| = (quotient
+// - 1) / (quotient + 1), in half the instructions of FP64 minima, maxima and
+// products. Roots are not negative; NaN passes through either path.
+struct LineSpread {
+  uint32_t lo_r, hi_r, lo_t, hi_t;
+  __device__ __forceinline__ LineSpread() : lo_r(~0u), hi_r(0), lo_t(~0u), hi_t(0) {}
+  __device__ __forceinline__ void add(double root_rho, double root_t) {
+    const uint32_t r = (uint32_t)(words(root_rho) >> 32), t = (uint32_t)(words(root_t) >> 32);
+    lo_r = min(lo_r, r);
+    hi_r = max(hi_r, r);
+    lo_t = min(lo_t, t);
+    hi_t = max(hi_t, t);
+  }
+  __device__ __forceinline__ bool far() const {
+    return max(hi_r - lo_r, hi_t - lo_t) > MeanSeries::max_spread;
+  }
+};
+
 // One line of direction O: volume terms added to acc. s_w, s_c: node records
-// and conservative states by variable; s_l: this lane's slots for logarithms
-// (FP64 flux_ranocha), NT apart. wend receives the records of the two end nodes
-// (FP32 flux_ranocha), pq the slots of the line's nodes.
-template <typename T, int D, int N, int VOL, int EPB, int NT, int O>
+// and conservative states by variable. wend receives the records of the two end
+// nodes (FP32 flux_ranocha), pq the slots of the line's nodes.
+template <typename T, int D, int N, int VOL, int EPB, int O>
 __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<T, N> &k, const LineCtx<T, D + 2> &c,
                                             const T *__restrict__ s_w, const T *__restrict__ s_c,
-                                            const double *__restrict__ s_alpha, T *__restrict__ s_l,
-                                            LineRecord<T, D, N> (&wend)[2], int (&pq)[N + 1],
+                                            const double *__restrict__ s_alpha, LineRecord<T, D, N> (&wend)[2], int (&pq)[N + 1],
                                             T (&acc)[N + 1][D + 2]) {
   using LY = Layout<D, N, EPB>;
   using VT = VolTraits<VOL>;
@@ -505,98 +525,69 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
       acc[i][V - 1] = tfma(k.Dsplit2[i * n + j], f[V - 1], acc[i][V - 1]);
       acc[j][V - 1] = tfma(k.Dsplit2[j * n + i], f[V - 1], acc[j][V - 1]);
     };
-    // Which form of the means the line takes. It depends on this line alone, so
-    // that results do not depend on the tile; the wavefront takes the cheapest
-    // path that serves all its lines. The high words h of two positive doubles
-    // order them, and their quotient is at most 1 + (h1 - h0) 2^-20 (the high word
-    // grows linearly within a binade, so per factor slowest at its start). So the
-    // largest minus the smallest high word of the line's roots bounds every
-    // pair's |f| = (quotient - 1) / (quotient + 1), in half the instructions of
-    // FP64 minima, maxima and products.
-    NodeD<D> w[n];
+    // Where all lines of the wavefront are in the range of the means' series no
+    // logarithms are taken, else two per node of the line (node_logs), and each pair of
+    // nodes selects for each mean. A pair's flux depends on the element alone, so that
+    // neither the path nor the tile shows in the results. Wavefronts with logarithms,
+    // every pair beyond the series: 3D p3 RHS on 32^3 elements 78 us, p4 on 16^3 31 us, 2D p3
+    // on 256^2 29 us (117, 50 and 47 us as a form per line, with both series, library
+    // logarithms and the pairs behind scheduling barriers; 94, 32 and 29 us with logarithms
+    // in every record). Logarithms shared through LDS by the workgroup, once per node, cost
+    // a barrier on the ordinary path, 3 % of the 2D p3 RHS, and gave nothing.
+    NodeD<D> x[n];
+    LineSpread sp;
 #pragma unroll
-    for (int i = 0; i < n; ++i) load_record<D, SZ>(w[i], s_w, pq[i]);
-    uint32_t lo_r = high_word(w[0].r), hi_r = lo_r, lo_t = high_word(w[0].t), hi_t = lo_t;
-#pragma unroll
-    for (int i = 1; i < n; ++i) {
-      const uint32_t r = high_word(w[i].r), t = high_word(w[i].t);
-      lo_r = min(lo_r, r);
-      hi_r = max(hi_r, r);
-      lo_t = min(lo_t, t);
-      hi_t = max(hi_t, t);
+    for (int i = 0; i < n; ++i) {
+      load_record<D, SZ>(x[i], s_w, pq[i]);
+      sp.add(x[i].r, x[i].t);
     }
-    const uint32_t sign = (hi_r | hi_t) & 0x80000000u;  // a negative value: logarithms, which give NaN
-    const uint32_t spread = max(max(hi_r - lo_r, hi_t - lo_t), sign);
+    // records read again (the opaque zero offset keeps the copies apart): held over the
+    // paths they would set the register allocation of the kernel
     auto fresh = [](const T *p) {
       int z0 = 0;
       asm volatile("" : "+v"(z0));
       return p + z0;
     };
-    const int kind = spread <= MeanSeriesShort::kMaxSpread  ? MEAN_SHORT
-                     : spread <= MeanSeriesLong::kMaxSpread ? MEAN_LONG
-                                                            : MEAN_LOG;
-    auto near_pairs = [&](const NodeD<D> (&x)[n]) {
-#pragma unroll
-      for (int i = 0; i < n; ++i)
-#pragma unroll
-        for (int j = i + 1; j < n; ++j) {
-          T f[V];
-          flux_ranocha_near<false, D, O>(x[i], x[j], kind, higm1, f);
-          add_pair(i, j, f);
-        }
-    };
-    if (__builtin_amdgcn_ballot_w64(kind != MEAN_SHORT) == 0) {
-      if constexpr (n <= 4) {
-        near_pairs(w);
-      } else {
-        // the records read again (the opaque zero offset keeps the copies apart):
-        // 141 us with, 153 us without (3D polydeg 4 RHS, 32^3 elements)
+    if (__builtin_amdgcn_ballot_w64(sp.far()) == 0) {
+      if constexpr (n > 4) {
         const T *sw = fresh(s_w);
-        NodeD<D> x[n];
 #pragma unroll
         for (int i = 0; i < n; ++i) load_record<D, SZ>(x[i], sw, pq[i]);
-        near_pairs(x);
       }
-    } else if (__builtin_amdgcn_ballot_w64(kind == MEAN_LOG) == 0) {
-      // each pair's records read again and the pairs kept in sequence (here and
-      // below): held or interleaved they would set the register allocation of
-      // the whole kernel
 #pragma unroll
       for (int i = 0; i < n; ++i)
 #pragma unroll
         for (int j = i + 1; j < n; ++j) {
           T f[V];
-          const T *sw = fresh(s_w);
-          NodeD<D> wi, wj;
-          load_record<D, SZ>(wi, sw, pq[i]);
-          load_record<D, SZ>(wj, sw, pq[j]);
-          flux_ranocha_near<true, D, O>(wi, wj, kind, higm1, f);
+          flux_ranocha_d<false, false, D, O>(x[i], x[j], T(0), T(0), higm1, f);
           add_pair(i, j, f);
-          __builtin_amdgcn_sched_barrier(0);
         }
     } else {
-      // Strong shocks: the logarithms of the line's roots, through LDS.
-#pragma unroll
-      for (int i = 0; i < n; ++i) {
-        const T *sw = fresh(s_w);
-        s_l[(2 * i) * NT] = Prec<T>::ln(sw[0 * SZ + pq[i]]);
-        s_l[(2 * i + 1) * NT] = Prec<T>::ln(sw[1 * SZ + pq[i]]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      // One after the other, with each node's records read anew, where the registers
+      // set the occupancy (flux differencing). Interleaved with shock capturing, whose kernels are at two
+      // wavefronts per SIMD either way (3D p4 on 16^3 elements 58 against 60 us).
+      constexpr bool ONE_BY_ONE = !VT::HG;
+      T ln_rho[n], ln_t[n];
+      const T *sw = fresh(s_w);
+      const int p0 = LY::phys(el * NN);
 #pragma unroll
       for (int i = 0; i < n; ++i)
+        node_logs(sw[pq[i]], sw[SZ + pq[i]], sw[p0], sw[SZ + p0], [](T y) { return Prec<T>::rcp(y); }, ln_rho[i],
+                  ln_t[i]);
+#pragma unroll
+      for (int i = 0; i < n; ++i) {
+        if constexpr (ONE_BY_ONE) sw = fresh(s_w);
+        NodeD<D> wi;
+        load_record<D, SZ>(wi, sw, pq[i]);
 #pragma unroll
         for (int j = i + 1; j < n; ++j) {
           T f[V];
-          const T *sw = fresh(s_w), *sl = fresh(s_l);
-          NodeD<D> wi, wj;
-          load_record<D, SZ>(wi, sw, pq[i]);
+          NodeD<D> wj;
           load_record<D, SZ>(wj, sw, pq[j]);
-          flux_ranocha_far<D, O>(wi, wj, kind, sl[(2 * i) * NT], sl[(2 * j) * NT], sl[(2 * i + 1) * NT],
-                                 sl[(2 * j + 1) * NT], higm1, f);
+          flux_ranocha_d<true, ONE_BY_ONE, D, O>(wi, wj, ln_rho[j] - ln_rho[i], ln_t[j] - ln_t[i], higm1, f);
           add_pair(i, j, f);
-          __builtin_amdgcn_sched_barrier(0);
         }
+      }
     }
   }
   if constexpr (VT::RAN && !F64) {
@@ -821,7 +812,7 @@ __device__ __forceinline__ void source_table_entry(const DGConst<T, N> &k, int i
 // phase B. In FP64 in 3D they take the records' memory too, the output tile
 // theirs after phase C, and a fused stage's epilogue has its scratch (node wave
 // speeds or indicator sums) at offset 0 and the new state behind it: 3D polydeg
-// 3 falls from 48 to 34 KB, three to four workgroups per CU, which the registers
+// 3 falls from 48 to 31 KB, three to four workgroups per CU, which the registers
 // allow. Elsewhere the records keep their own memory, where the output tile goes
 // without the barrier and the registers that the shared one costs (FP32 3D p3
 // RHS 26.2 against 25.1 us; 2D meshes do not fill the chip).
@@ -844,15 +835,11 @@ template <typename T, int D, int N, int VOL, int EPB, int WPD, int MODE> struct 
       max2((size_t)D * NQ * sizeof(double), IND2D ? (size_t)(EPB / 16) * 512 * sizeof(double) : 0);
   static constexpr size_t NEW = STAGE ? align16((size_t)NQ * V * sizeof(double)) : 0;  // new state of a fused stage
   static constexpr bool SHARE = sizeof(T) == 8 && D == 3;
-  // logarithms behind the records, or between the tile and them
-  static constexpr size_t LOGS =
-      VolTraits<VOL>::RAN && sizeof(T) == 8 ? (size_t)2 * (N + 1) * D * WPD * 64 * sizeof(T) : 0;
-  static constexpr size_t OFF_RECORDS = SHARE ? TILE : align16(max2(max2(TILE + LOGS, LINES), NEW));
-  static constexpr size_t OFF_LOGS = SHARE ? TILE + RECORDS : TILE;
+  static constexpr size_t OFF_RECORDS = SHARE ? TILE : align16(max2(LINES, NEW));
   static constexpr size_t OFF_OUT = SHARE ? 0 : OFF_RECORDS;  // output tile, later the epilogue's scratch
   static constexpr size_t OFF_NEW = SHARE ? align16(max2(TILE, SCRATCH)) : 0;
   static constexpr size_t BYTES =
-      SHARE ? align16(max2(max2(TILE + RECORDS + LOGS, LINES), STAGE ? OFF_NEW + NEW : 0))
+      SHARE ? align16(max2(max2(TILE + RECORDS, LINES), STAGE ? OFF_NEW + NEW : 0))
             : OFF_RECORDS + max2(max2(RECORDS, TILE), STAGE ? SCRATCH : 0);
 };
 
@@ -933,10 +920,10 @@ __device__ __forceinline__ void stage_indicator_2d(const ElemArgs<T> &a, const d
 // into registers), the per-element scalars, then the neighbour face states,
 // which stay in flight until phase B.
 // Minimum wavefronts per SIMD the register allocation must allow: the FP64 3D
-// flux_ranocha variants are held to 168 VGPRs, which their means without
-// logarithms meet; the rarely run ones with logarithms spill a few values.
+// flux_ranocha variants are held to 168 VGPRs with flux differencing and to 256 with
+// shock capturing, which they meet without scratch memory.
 template <typename T, int D, int N, int VOL> constexpr int min_waves_per_simd() {
-  return sizeof(T) == 8 && D == 3 && VOL == VOL_FD_RANOCHA ? 3 : 1;
+  return sizeof(T) == 8 && D == 3 && VolTraits<VOL>::RAN ? (VOL == VOL_FD_RANOCHA ? 3 : 2) : 1;
 }
 
 template <typename T, int D, int N, int VOL, int EPB, int WPD, bool BND, int MODE>
@@ -961,7 +948,6 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
   T *s_t = reinterpret_cast<T *>(smem);                     // staged tile [EPB*NN][V]
   T *s_w = reinterpret_cast<T *>(smem + LDS::OFF_RECORDS);  // [NW][SZ]
   T *s_c = s_w + LDS::NW * SZ;                              // [NC][SZ]
-  T *s_l = reinterpret_cast<T *>(smem + LDS::OFF_LOGS);     // [2 n][NT] logarithms (FP64 flux_ranocha)
   T *s_d = reinterpret_cast<T *>(smem);                     // [D][V][SZ] line results, after phase B
   T *s_o = reinterpret_cast<T *>(smem + LDS::OFF_OUT);      // [EPB*NN][V] output, after phase C
 
@@ -1120,7 +1106,7 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
   };
   if (lc.valid) {
     in_direction([&](auto o) {
-      line_volume<T, D, N, VOL, EPB, NT, o.value>(a, k, lc, s_w, s_c, s_alpha, s_l + tid, wend, pq, acc);
+      line_volume<T, D, N, VOL, EPB, o.value>(a, k, lc, s_w, s_c, s_alpha, wend, pq, acc);
       // keep the face work (which waits on the neighbour loads of phase A)
       // behind the volume arithmetic
       __builtin_amdgcn_sched_barrier(0);
