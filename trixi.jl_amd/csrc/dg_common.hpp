@@ -264,18 +264,18 @@ __device__ __forceinline__ void flux_ranocha_fast(const NodeR<float, D> &l, cons
   f[D + 1] = tfma(f1, inner_h, cross);  // half the energy flux
 }
 
-// Per-node data of the FP64 flux_ranocha lines: the roots r of the density and
-// t of the temperature T = p/rho (1/T is the beta of the means above, and
-// sqrt(gamma) t the sound speed), half velocities, half pressure. No logarithms
-// are stored: two per node cost more than the series of log_means, and the
-// line's records take fewer registers (three wavefronts per SIMD for polydeg 3
-// and 4 in 3D).
+// Per-node data of the FP64 flux_ranocha lines: density, temperature T = p/rho (1/T
+// is the beta of the means above), half velocities, half pressure. The record in LDS
+// has sqrt(T) too (sound speed sqrt(gamma) sqrt(T)), which the surface and subcell
+// fluxes read. No logarithms are stored: two per node cost more than the series
+// of log_means, which serves where neighbouring nodes do not differ much.
 template <int D> struct NodeD {
   double r, t, h[D], hp;
 };
-template <typename T, int D> constexpr int node_record_size() { return sizeof(T) == 8 ? 3 + D : nodeR_count(D); }
+template <typename T, int D> constexpr int node_record_size() { return sizeof(T) == 8 ? 4 + D : nodeR_count(D); }
 
-template <int D> __device__ __forceinline__ void nodeD_from_cons(const double *u, double gamma_m1, NodeD<D> &w) {
+template <int D>
+__device__ __forceinline__ void nodeD_from_cons(const double *u, double gamma_m1, NodeD<D> &w, double &root_t) {
   const double irho = Prec<double>::rcp(u[0]);
   double ke2 = 0, v[D];
 #pragma unroll
@@ -285,8 +285,9 @@ template <int D> __device__ __forceinline__ void nodeD_from_cons(const double *u
     w.h[d] = 0.5 * v[d];
   }
   const double p = gamma_m1 * (u[D + 1] - 0.5 * ke2);
-  w.r = Prec<double>::sqrt_(u[0]);
-  w.t = Prec<double>::sqrt_(p * irho);
+  w.r = u[0];
+  w.t = p * irho;
+  root_t = Prec<double>::sqrt_(w.t);
   w.hp = 0.5 * p;
 }
 
@@ -410,17 +411,17 @@ __device__ __forceinline__ void consp_from_node(const float *u, const NodeR<floa
   cs = sqrt_gamma * w.b;
 }
 
-// The same for an FP64 line: v = 2 h, p = 2 hp, sound speed sqrt(gamma) t.
+// The same for an FP64 line: v = 2 h, p = 2 hp, sound speed sqrt(gamma) sqrt(T).
 template <int D>
-__device__ __forceinline__ void consp_from_node(const double *u, const NodeD<D> &w, double sqrt_gamma, ConsP<double, D> &c,
-                                                double &cs) {
+__device__ __forceinline__ void consp_from_node(const double *u, const NodeD<D> &w, double root_t, double sqrt_gamma,
+                                                ConsP<double, D> &c, double &cs) {
 #pragma unroll
   for (int k = 0; k < D + 2; ++k) c.u[k] = u[k];
 #pragma unroll
   for (int d = 0; d < D; ++d) c.v[d] = 2.0 * w.h[d];
   c.p = 2.0 * w.hp;
   c.irho = 0.0;  // not needed by phys_flux / flux_llf_pc
-  cs = sqrt_gamma * w.t;
+  cs = sqrt_gamma * root_t;
 }
 
 // FluxLaxFriedrichs(max_abs_speed | max_abs_speed_naive)

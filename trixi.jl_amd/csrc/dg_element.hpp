@@ -359,6 +359,9 @@ template <int D, int SZ> __device__ __forceinline__ void load_record(NodeD<D> &x
   for (int d = 0; d < D; ++d) x.h[d] = s_w[(2 + d) * SZ + q];
   x.hp = s_w[(2 + D) * SZ + q];
 }
+template <int D, int SZ> __device__ __forceinline__ double load_root_t(const double *s_w, int q) {
+  return s_w[(3 + D) * SZ + q];
+}
 
 template <typename T, int D, int N, int VOL, int EPB, int O, bool BND>
 __device__ __forceinline__ void line_faces(const ElemArgs<T> &a, const DGConst<T, N> &k, const LineCtx<T, D + 2> &c,
@@ -395,11 +398,15 @@ __device__ __forceinline__ void line_faces(const ElemArgs<T> &a, const DGConst<T
       ConsP<T, D> own_face[2];
       T own_c[2];
       if constexpr (F64) {
-        load_record<D, SZ>(wend[0], s_w, LY::phys(q0));
-        load_record<D, SZ>(wend[1], s_w, LY::phys(q0 + (n - 1) * st));
+        const int p0 = LY::phys(q0), p1 = LY::phys(q0 + (n - 1) * st);
+        load_record<D, SZ>(wend[0], s_w, p0);
+        load_record<D, SZ>(wend[1], s_w, p1);
+        consp_from_node<D>(own0, wend[0], load_root_t<D, SZ>(s_w, p0), a.sqrt_gamma, own_face[0], own_c[0]);
+        consp_from_node<D>(own1, wend[1], load_root_t<D, SZ>(s_w, p1), a.sqrt_gamma, own_face[1], own_c[1]);
+      } else {
+        consp_from_node<D>(own0, wend[0], a.sqrt_gamma, own_face[0], own_c[0]);
+        consp_from_node<D>(own1, wend[1], a.sqrt_gamma, own_face[1], own_c[1]);
       }
-      consp_from_node<D>(own0, wend[0], a.sqrt_gamma, own_face[0], own_c[0]);
-      consp_from_node<D>(own1, wend[1], a.sqrt_gamma, own_face[1], own_c[1]);
       // twice the LLF flux with half the weight (bitwise the same terms);
       // a given mortar flux is doubled to match
       const T hfactor = T(0.5) * factor;
@@ -448,21 +455,21 @@ __device__ __forceinline__ void line_faces(const ElemArgs<T> &a, const DGConst<T
 // means' series. The high words h of two positive doubles order them, and their
 // quotient is at most 1 + (h1 - h0) 2^-20 while that is below 2 (the high word grows
 // linearly within a binade, so per factor slowest at its start). So the largest minus
-// the smallest high word of the line's roots bounds every pair's |f| = (quotient
-// - 1) / (quotient + 1), in half the instructions of FP64 minima, maxima and
-// products. Roots are not negative; NaN passes through either path.
+// the smallest high word of the line's values bounds every pair's quotient, in half
+// the instructions of FP64 minima, maxima and products. A negative value sets the
+// high bit: it goes to the logarithms, which give NaN.
 struct LineSpread {
   uint32_t lo_r, hi_r, lo_t, hi_t;
   __device__ __forceinline__ LineSpread() : lo_r(~0u), hi_r(0), lo_t(~0u), hi_t(0) {}
-  __device__ __forceinline__ void add(double root_rho, double root_t) {
-    const uint32_t r = (uint32_t)(words(root_rho) >> 32), t = (uint32_t)(words(root_t) >> 32);
+  __device__ __forceinline__ void add(double rho, double temperature) {
+    const uint32_t r = high_word(rho), t = high_word(temperature);
     lo_r = min(lo_r, r);
     hi_r = max(hi_r, r);
     lo_t = min(lo_t, t);
     hi_t = max(hi_t, t);
   }
   __device__ __forceinline__ bool far() const {
-    return max(hi_r - lo_r, hi_t - lo_t) > MeanSeries::max_spread;
+    return max(max(hi_r - lo_r, hi_t - lo_t), (hi_r | hi_t) & 0x80000000u) > MeanSeries::max_spread;
   }
 };
 
@@ -564,7 +571,8 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
         }
     } else {
       // One after the other, with each node's records read anew, where the registers
-      // set the occupancy (flux differencing). Interleaved with shock capturing, whose kernels are at two
+      // set the occupancy (flux differencing: 3D p3 near path 59 against 65 us, the pairs
+      // interleaved). Interleaved with shock capturing, whose kernels are at two
       // wavefronts per SIMD either way (3D p4 on 16^3 elements 58 against 60 us).
       constexpr bool ONE_BY_ONE = !VT::HG;
       T ln_rho[n], ln_t[n];
@@ -731,7 +739,7 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
         if (llf) {
           NodeD<D> w0;
           load_record<D, SZ>(w0, s_w, pq[0]);
-          consp_from_node<D>(cur, w0, a.sqrt_gamma, pcur, ccur);
+          consp_from_node<D>(cur, w0, load_root_t<D, SZ>(s_w, pq[0]), a.sqrt_gamma, pcur, ccur);
         }
       }
 #pragma unroll
@@ -745,7 +753,7 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
 #pragma unroll
             for (int v = 0; v < V; ++v) nxt[v] = s_c[v * SZ + pq[i + 1]];
             load_record<D, SZ>(w1, s_w, pq[i + 1]);
-            consp_from_node<D>(nxt, w1, a.sqrt_gamma, pnxt, cnxt);
+            consp_from_node<D>(nxt, w1, load_root_t<D, SZ>(s_w, pq[i + 1]), a.sqrt_gamma, pnxt, cnxt);
             flux_llf_pc<T, D, O>(pcur, pnxt, ccur, cnxt, a.fv_flux == FLUX_LLF_NAIVE, fnext);
             pcur = pnxt;
             ccur = cnxt;
@@ -1068,12 +1076,14 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
       }
       if constexpr (VT::RAN && sizeof(T) == 8) {
         NodeD<D> w;
-        nodeD_from_cons<D>(uq, gm1, w);
+        double root_t;
+        nodeD_from_cons<D>(uq, gm1, w, root_t);
         s_w[0 * SZ + p] = w.r;
         s_w[1 * SZ + p] = w.t;
 #pragma unroll
         for (int d = 0; d < D; ++d) s_w[(2 + d) * SZ + p] = w.h[d];
         s_w[(2 + D) * SZ + p] = w.hp;
+        s_w[(3 + D) * SZ + p] = root_t;
       }
       if constexpr (VT::RAN && sizeof(T) == 4) {
         NodeR<T, D> w;
