@@ -25,8 +25,9 @@ void means(int n, const double *rl, const double *rr, const double *tl, const do
     double a, b, c, d;
     node_logs(rl[i], tl[i], r0[i], t0[i], rcp, a, b);
     node_logs(rr[i], tr[i], r0[i], t0[i], rcp, c, d);
-    log_means<true, false>(rl[i], rr[i], tl[i], tr[i], c - a, d - b, rcp, rho[i], inv[i]);
-    log_means<false, false>(rl[i], rr[i], tl[i], tr[i], 0.0, 0.0, rcp, rho_series[i], inv_series[i]);
+    const double x = 0.5 * rl[i], y = 0.5 * rr[i], s = 0.5 * tl[i], t = 0.5 * tr[i];
+    log_means<true, false>(x, y, s, t, c - a, d - b, rcp, rho[i], inv[i]);
+    log_means<false, false>(x, y, s, t, 0.0, 0.0, rcp, rho_series[i], inv_series[i]);
   }
 }
 void logs(int n, const double *x, const double *x0, double *out) {
@@ -91,17 +92,17 @@ def draw(rng, n, lo, hi, scale):
 
 # In units of 2^-53. Series: the sum of the two values and the last multiply-add, two roundings, rms 0.43 each of a
 # value whose mantissa is spread evenly over its logarithm, 0.60 together, largest 2; the series' own part is
-# below 4 % of the mean, with a few roundings of its own.
+# below 5 % of the mean, with a few roundings of its own.
 NEAR_RMS, NEAR_MAX = 0.75, 2.25
 # Logarithms: y - x, the corrected quotient, the difference of the logarithms 1 each at most; each
-# logarithm |l| / |L| <= 1.2 of its own rounding and 2.5 of s on at most 0.41 / 0.405 of L; the
+# logarithm |l| / |L| <= 1.2 of its own rounding and 2.5 of s on at most 0.41 / 0.53 of L; the
 # temperature's product and its last product 1 each.
 FAR_MAX, FAR_RMS = 13.0, 2.5
 
 
 @pytest.mark.parametrize("scale", [1.0, 1e-7, 1e5])
-@pytest.mark.parametrize("lo,hi", [(1e-12, 1e-9), (1e-9, 1e-4), (1e-4, 0.02), (0.02, 0.1), (0.1, 0.5), (0.5, 0.83),
-                                   (0.83, 3.0), (3.0, 100.0), (100.0, 1e8)])
+@pytest.mark.parametrize("lo,hi", [(1e-12, 1e-9), (1e-9, 1e-4), (1e-4, 0.02), (0.02, 0.1), (0.1, 0.69),
+                                   (0.71, 3.0), (3.0, 100.0), (100.0, 1e8)])
 def test_means_against_exact_values(lib, lo, hi, scale):
     rng = np.random.default_rng(int(1e6 * hi) % 1000003)
     n = 1500
@@ -110,7 +111,7 @@ def test_means_against_exact_values(lib, lo, hi, scale):
     rho, inv, _, _ = means(lib, rl, rr, tl, tr, r0, t0)
     e_rho = np.array([float((Decimal(float(a)) - m) / m) for a, m in zip(rho, (exact_means(x, y)[0] for x, y in zip(rl, rr)))])
     e_inv = np.array([float((Decimal(float(a)) - m) / m) for a, m in zip(inv, (exact_means(x, y)[1] for x, y in zip(tl, tr)))])
-    near = hi <= 0.5
+    near = hi < 0.7
     for name, e in (("density", e_rho / UNIT), ("temperature", e_inv / UNIT)):
         rms, big = float(np.sqrt(np.mean(e * e))), float(np.max(np.abs(e)))
         print(f"{name} 1+[{lo:g}, {hi:g}] scale {scale:g}: rms {rms:.2f} largest {big:.2f}")
@@ -147,13 +148,14 @@ def test_range_is_taken_alike_on_both_paths(lib):
     assert (q - 1) / (q + 1) <= f
 
 
-@pytest.mark.parametrize("which,stated", [(0, 1.1e-17), (1, 7.6e-18), (2, 7.6e-19)])
+@pytest.mark.parametrize("which,stated", [(0, 1.3e-17), (1, 1.1e-17), (2, 7.6e-19)])
 def test_series_coefficients(lib, which, stated):
     """Largest relative error of m (1 + z S), m (1 + z R) and 1 + z P over their range, from the coefficients as
     they are: one that is off in its last places shows."""
     c = (ctypes.c_double * 32)()
     c = [Decimal(v) for v in c[:lib.series(which, c)]]
-    top = Decimal("0.2") ** 2
+    top = Decimal("0.2") if which == 2 else Decimal("0.7") / Decimal("2.7")
+    top = top * top
     worst = Decimal(0)
     for i in range(1, 301):
         z = top * i / 300

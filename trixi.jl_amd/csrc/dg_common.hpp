@@ -264,18 +264,16 @@ __device__ __forceinline__ void flux_ranocha_fast(const NodeR<float, D> &l, cons
   f[D + 1] = tfma(f1, inner_h, cross);  // half the energy flux
 }
 
-// Per-node data of the FP64 flux_ranocha lines: density, temperature T = p/rho (1/T
-// is the beta of the means above), half velocities, half pressure. The record in LDS
-// has sqrt(T) too (sound speed sqrt(gamma) sqrt(T)), which the surface and subcell
-// fluxes read. No logarithms are stored: two per node cost more than the series
+// Per-node data of the FP64 flux_ranocha lines: halves of density, temperature T = p/rho
+// (1/T is the beta of the means above), velocities and pressure. No logarithms are stored: two per node cost more than the series
 // of log_means, which serves where neighbouring nodes do not differ much.
 template <int D> struct NodeD {
-  double r, t, h[D], hp;
+  double hr, ht, h[D], hp;
 };
-template <typename T, int D> constexpr int node_record_size() { return sizeof(T) == 8 ? 4 + D : nodeR_count(D); }
+template <typename T, int D> constexpr int node_record_size() { return sizeof(T) == 8 ? 3 + D : nodeR_count(D); }
 
 template <int D>
-__device__ __forceinline__ void nodeD_from_cons(const double *u, double gamma_m1, NodeD<D> &w, double &root_t) {
+__device__ __forceinline__ void nodeD_from_cons(const double *u, double gamma_m1, NodeD<D> &w) {
   const double irho = Prec<double>::rcp(u[0]);
   double ke2 = 0, v[D];
 #pragma unroll
@@ -285,9 +283,8 @@ __device__ __forceinline__ void nodeD_from_cons(const double *u, double gamma_m1
     w.h[d] = 0.5 * v[d];
   }
   const double p = gamma_m1 * (u[D + 1] - 0.5 * ke2);
-  w.r = u[0];
-  w.t = p * irho;
-  root_t = Prec<double>::sqrt_(w.t);
+  w.hr = 0.5 * u[0];
+  w.ht = 0.5 * (p * irho);
   w.hp = 0.5 * p;
 }
 
@@ -315,7 +312,7 @@ template <bool LOGS, bool ORDERED, int D, int O>
 __device__ __forceinline__ void flux_ranocha_d(const NodeD<D> &l, const NodeD<D> &r, double ln_rho, double ln_t,
                                                double half_inv_gamma_m1, double *f) {
   double rho_mean, inv_rho_p_mean;
-  log_means<LOGS, ORDERED>(l.r, r.r, l.t, r.t, ln_rho, ln_t, [](double x) { return Prec<double>::rcp(x); }, rho_mean,
+  log_means<LOGS, ORDERED>(l.hr, r.hr, l.ht, r.ht, ln_rho, ln_t, [](double x) { return Prec<double>::rcp(x); }, rho_mean,
                            inv_rho_p_mean);
   flux_ranocha_tail<D, O>(l, r, rho_mean, inv_rho_p_mean, half_inv_gamma_m1, f);
 }

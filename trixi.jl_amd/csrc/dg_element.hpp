@@ -352,15 +352,25 @@ template <int D, int N, int EPB, int O> __device__ __forceinline__ void line_slo
 // the records of the two end nodes: wend (read here in FP64).
 template <typename T, int D, int N> using LineRecord = std::conditional_t<sizeof(T) == 8, NodeD<D>, NodeR<T, D>>;
 
-template <int D, int SZ> __device__ __forceinline__ void load_record(NodeD<D> &x, const double *s_w, int q) {
-  x.r = s_w[0 * SZ + q];
-  x.t = s_w[1 * SZ + q];
+// FP64 records: [hr or sqrt(T)][ht][h][hp]. With shock capturing, whose subcell fluxes
+// take a sound speed at every node, row 0 is sqrt(T), and the density comes from the
+// conservative states behind the records; flux differencing takes the root at its two
+// faces. One more row would cost the 2D p3 stage its fourth workgroup per CU (200 steps of
+// the Kelvin-Helmholtz solve on 128^2 elements 24.4 ms instead of 18.8).
+template <int D, int SZ, bool HG> __device__ __forceinline__ double load_hr(const double *s_w, int q) {
+  if constexpr (HG) return 0.5 * s_w[node_record_size<double, D>() * SZ + q];
+  else return s_w[q];
+}
+template <int D, int SZ, bool HG> __device__ __forceinline__ double load_root_t(const double *s_w, int q) {
+  if constexpr (HG) return s_w[q];
+  else return Prec<double>::sqrt_(2.0 * s_w[SZ + q]);
+}
+template <int D, int SZ, bool HG> __device__ __forceinline__ void load_record(NodeD<D> &x, const double *s_w, int q) {
+  x.hr = load_hr<D, SZ, HG>(s_w, q);
+  x.ht = s_w[1 * SZ + q];
 #pragma unroll
   for (int d = 0; d < D; ++d) x.h[d] = s_w[(2 + d) * SZ + q];
   x.hp = s_w[(2 + D) * SZ + q];
-}
-template <int D, int SZ> __device__ __forceinline__ double load_root_t(const double *s_w, int q) {
-  return s_w[(3 + D) * SZ + q];
 }
 
 template <typename T, int D, int N, int VOL, int EPB, int O, bool BND>
@@ -399,10 +409,10 @@ __device__ __forceinline__ void line_faces(const ElemArgs<T> &a, const DGConst<T
       T own_c[2];
       if constexpr (F64) {
         const int p0 = LY::phys(q0), p1 = LY::phys(q0 + (n - 1) * st);
-        load_record<D, SZ>(wend[0], s_w, p0);
-        load_record<D, SZ>(wend[1], s_w, p1);
-        consp_from_node<D>(own0, wend[0], load_root_t<D, SZ>(s_w, p0), a.sqrt_gamma, own_face[0], own_c[0]);
-        consp_from_node<D>(own1, wend[1], load_root_t<D, SZ>(s_w, p1), a.sqrt_gamma, own_face[1], own_c[1]);
+        load_record<D, SZ, VT::HG>(wend[0], s_w, p0);
+        load_record<D, SZ, VT::HG>(wend[1], s_w, p1);
+        consp_from_node<D>(own0, wend[0], load_root_t<D, SZ, VT::HG>(s_w, p0), a.sqrt_gamma, own_face[0], own_c[0]);
+        consp_from_node<D>(own1, wend[1], load_root_t<D, SZ, VT::HG>(s_w, p1), a.sqrt_gamma, own_face[1], own_c[1]);
       } else {
         consp_from_node<D>(own0, wend[0], a.sqrt_gamma, own_face[0], own_c[0]);
         consp_from_node<D>(own1, wend[1], a.sqrt_gamma, own_face[1], own_c[1]);
@@ -545,8 +555,8 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
     LineSpread sp;
 #pragma unroll
     for (int i = 0; i < n; ++i) {
-      load_record<D, SZ>(x[i], s_w, pq[i]);
-      sp.add(x[i].r, x[i].t);
+      load_record<D, SZ, VT::HG>(x[i], s_w, pq[i]);
+      sp.add(x[i].hr, x[i].ht);
     }
     // records read again (the opaque zero offset keeps the copies apart): held over the
     // paths they would set the register allocation of the kernel
@@ -559,7 +569,7 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
       if constexpr (n > 4) {
         const T *sw = fresh(s_w);
 #pragma unroll
-        for (int i = 0; i < n; ++i) load_record<D, SZ>(x[i], sw, pq[i]);
+        for (int i = 0; i < n; ++i) load_record<D, SZ, VT::HG>(x[i], sw, pq[i]);
       }
 #pragma unroll
       for (int i = 0; i < n; ++i)
@@ -580,18 +590,18 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
       const int p0 = LY::phys(el * NN);
 #pragma unroll
       for (int i = 0; i < n; ++i)
-        node_logs(sw[pq[i]], sw[SZ + pq[i]], sw[p0], sw[SZ + p0], [](T y) { return Prec<T>::rcp(y); }, ln_rho[i],
-                  ln_t[i]);
+        node_logs(load_hr<D, SZ, VT::HG>(sw, pq[i]), sw[SZ + pq[i]], load_hr<D, SZ, VT::HG>(sw, p0), sw[SZ + p0],
+                  [](T y) { return Prec<T>::rcp(y); }, ln_rho[i], ln_t[i]);
 #pragma unroll
       for (int i = 0; i < n; ++i) {
         if constexpr (ONE_BY_ONE) sw = fresh(s_w);
         NodeD<D> wi;
-        load_record<D, SZ>(wi, sw, pq[i]);
+        load_record<D, SZ, VT::HG>(wi, sw, pq[i]);
 #pragma unroll
         for (int j = i + 1; j < n; ++j) {
           T f[V];
           NodeD<D> wj;
-          load_record<D, SZ>(wj, sw, pq[j]);
+          load_record<D, SZ, VT::HG>(wj, sw, pq[j]);
           flux_ranocha_d<true, ONE_BY_ONE, D, O>(wi, wj, ln_rho[j] - ln_rho[i], ln_t[j] - ln_t[i], higm1, f);
           add_pair(i, j, f);
         }
@@ -738,8 +748,8 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
       if constexpr (FROM_W) {
         if (llf) {
           NodeD<D> w0;
-          load_record<D, SZ>(w0, s_w, pq[0]);
-          consp_from_node<D>(cur, w0, load_root_t<D, SZ>(s_w, pq[0]), a.sqrt_gamma, pcur, ccur);
+          load_record<D, SZ, VT::HG>(w0, s_w, pq[0]);
+          consp_from_node<D>(cur, w0, load_root_t<D, SZ, VT::HG>(s_w, pq[0]), a.sqrt_gamma, pcur, ccur);
         }
       }
 #pragma unroll
@@ -752,8 +762,8 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
             T nxt[V], cnxt;
 #pragma unroll
             for (int v = 0; v < V; ++v) nxt[v] = s_c[v * SZ + pq[i + 1]];
-            load_record<D, SZ>(w1, s_w, pq[i + 1]);
-            consp_from_node<D>(nxt, w1, load_root_t<D, SZ>(s_w, pq[i + 1]), a.sqrt_gamma, pnxt, cnxt);
+            load_record<D, SZ, VT::HG>(w1, s_w, pq[i + 1]);
+            consp_from_node<D>(nxt, w1, load_root_t<D, SZ, VT::HG>(s_w, pq[i + 1]), a.sqrt_gamma, pnxt, cnxt);
             flux_llf_pc<T, D, O>(pcur, pnxt, ccur, cnxt, a.fv_flux == FLUX_LLF_NAIVE, fnext);
             pcur = pnxt;
             ccur = cnxt;
@@ -1076,14 +1086,12 @@ void dg_element_kernel(ElemArgs<T> a, DGConst<T, N> k) {
       }
       if constexpr (VT::RAN && sizeof(T) == 8) {
         NodeD<D> w;
-        double root_t;
-        nodeD_from_cons<D>(uq, gm1, w, root_t);
-        s_w[0 * SZ + p] = w.r;
-        s_w[1 * SZ + p] = w.t;
+        nodeD_from_cons<D>(uq, gm1, w);
+        s_w[0 * SZ + p] = VT::HG ? Prec<T>::sqrt_(T(2) * w.ht) : w.hr;
+        s_w[1 * SZ + p] = w.ht;
 #pragma unroll
         for (int d = 0; d < D; ++d) s_w[(2 + d) * SZ + p] = w.h[d];
         s_w[(2 + D) * SZ + p] = w.hp;
-        s_w[(3 + D) * SZ + p] = root_t;
       }
       if constexpr (VT::RAN && sizeof(T) == 4) {
         NodeR<T, D> w;
