@@ -176,7 +176,7 @@ struct trixi_hip_ctx {
   // element-kernel launch (elem_stage: the variant with the fused 2N update,
   // null when not instantiated for the tile or switched off); each with its
   // own tile (elements per workgroup, threads)
-  ElemLaunch elem = nullptr, elem_stage = nullptr;
+  ElemLaunch elem = nullptr, elem_rhs64 = nullptr, elem_stage = nullptr;  // elem_rhs64: FP32, between FP64 arrays
   int epb = 0, nt = 0, epb_st = 0, nt_st = 0;
   std::vector<unsigned char> kconst;  // DGConst<T, N> blob
   // workgroups of the element kernel walk contiguous element ranges per XCD
@@ -455,6 +455,7 @@ int select_tile(trixi_hip_ctx *ctx, int epb, int nt) {
                    "integral, tile, boundaries)");
   const char *unfused = std::getenv("TRIXI_HIP_UNFUSED_STAGE");
   ctx->elem_stage = (unfused && std::atoi(unfused) != 0) ? nullptr : find_launch(ctx, 1, e_s, n_s);
+  ctx->elem_rhs64 = find_launch(ctx, ELEM_RHS64, e_r, n_r);
   ctx->epb = e_r;
   ctx->nt = n_r;
   ctx->epb_st = ctx->elem_stage ? e_s : 0;
@@ -677,8 +678,8 @@ int launch_rhs_T(trixi_hip_ctx *ctx, T *du, const T *u, double t, const double *
   a.gamma64 = ctx->cfg.gamma;
   const int epb = so ? ctx->epb_st : ctx->epb;
   int nblocks = (ctx->E + epb - 1) / epb;
-  ElemLaunch launch = so ? ctx->elem_stage : ctx->elem;
-  if (du64 && !(launch = find_launch(ctx, ELEM_RHS64, ctx->epb, ctx->nt)))
+  const ElemLaunch launch = so ? ctx->elem_stage : du64 ? ctx->elem_rhs64 : ctx->elem;
+  if (!launch)
     return set_err(ctx, TRIXI_HIP_EINVAL, "no element kernel between FP64 arrays for this tile");
   hipError_t e = launch(&a, ctx->kconst.data(), nblocks, ctx->stream);
   if (e != hipSuccess) return set_err(ctx, TRIXI_HIP_EHIP, std::string("element kernel launch: ") + hipGetErrorString(e));
@@ -1026,7 +1027,7 @@ int trixi_hip_create(const trixi_hip_config *cfg, const trixi_hip_mesh *mesh,
   ctx->stream = ctx->own_stream;
   const size_t nv = ctx->nvals;
   const size_t tsz = ctx->fp32 ? 4 : 8;
-  ctx->partial_cap = std::max<size_t>((size_t)E * 2 * ctx->V, kMaxPartials);
+  ctx->partial_cap = std::max<size_t>((size_t)E, kMaxPartials);  // one per tile of the wave speed at most
   bool ok = dev_alloc(ctx, &ctx->d_nbr, nbr.size() * 4) == hipSuccess &&
             dev_alloc(ctx, &ctx->d_invj, E * 8) == hipSuccess &&
             dev_alloc(ctx, &ctx->d_centers, (size_t)D * E * 8) == hipSuccess &&
@@ -2074,6 +2075,7 @@ int trixi_hip_autotune(trixi_hip_ctx *ctx, int repetitions, trixi_hip_tile_timin
     if (!best) continue;
     if (stage == 0) {
       ctx->elem = best->fn;
+      ctx->elem_rhs64 = find_launch(ctx, ELEM_RHS64, best->epb, best->nt);
       ctx->epb = best->epb;
       ctx->nt = best->nt;
     } else {
