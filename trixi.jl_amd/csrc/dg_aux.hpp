@@ -649,9 +649,9 @@ __global__ __launch_bounds__(256) void integrals_kernel(const double *__restrict
 }
 
 // Column blockIdx.x of a partial table [rows, cols] -> out: its sum, or its
-// maximum (NaN wins) for columns from nsum on. One workgroup for each column: 5 us
-// for 937 rows of 10 columns or 2048 of 6. One workgroup for all columns, a row for each
-// of 32 768 elements: 216 and 118 us.
+// maximum (NaN wins) for columns from nsum on. One workgroup for each column: 5.2 us
+// for 729 rows of 10 columns or 2048 of 6 (3D p3 on 32^3 elements). One workgroup for all
+// columns, a row for each of 32 768 elements: 216 and 118 us.
 static __global__ __launch_bounds__(256) void reduce_columns_kernel(const double *__restrict__ partial, int rows,
                                                                     int cols, int nsum, double *__restrict__ out) {
   __shared__ double s_red[4];

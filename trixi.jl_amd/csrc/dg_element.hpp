@@ -149,8 +149,8 @@ template <typename T, int D, int N, int EPB> struct TileIO {
 // W consecutive values between global memory (aligned to the smaller of 16 and
 // W sizeof(S) bytes) and registers, in pieces of up to 16 bytes. A fused stage
 // that moved its registers value by value, 4 and 8 bytes at strides of 16 and 32,
-// was bound by the number of its memory accesses: FP32 3D p3 stage 70.4 -> 54 us,
-// FP64 98 -> 90 us (32^3 elements; 252 and 420 MB).
+// was bound by the number of its memory accesses: FP32 3D p3 stage kernel 70.4 -> 53 us,
+// FP64 98 -> 90 us (32^3 elements; 252 and 336 MB).
 template <typename S, int W> struct Pieces {
   static constexpr int K = 16 / (int)sizeof(S) < W ? 16 / (int)sizeof(S) : W;
   typedef S V __attribute__((ext_vector_type(K > 1 ? K : 2)));
@@ -546,7 +546,7 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
     // logarithms are taken, else two per node of the line (node_logs), and each pair of
     // nodes selects for each mean. A pair's flux depends on the element alone, so that
     // neither the path nor the tile shows in the results. Wavefronts with logarithms,
-    // every pair beyond the series: 3D p3 RHS on 32^3 elements 78 us, p4 on 16^3 31 us, 2D p3
+    // every pair beyond the series: 3D p3 RHS on 32^3 elements 75 us, p4 on 16^3 30 us, 2D p3
     // on 256^2 29 us (117, 50 and 47 us as a form per line, with both series, library
     // logarithms and the pairs behind scheduling barriers; 94, 32 and 29 us with logarithms
     // in every record). Logarithms shared through LDS by the workgroup, once per node, cost
@@ -583,7 +583,7 @@ __device__ __forceinline__ void line_volume(const ElemArgs<T> &a, const DGConst<
       // One after the other, with each node's records read anew, where the registers
       // set the occupancy (flux differencing: 3D p3 near path 59 against 65 us, the pairs
       // interleaved). Interleaved with shock capturing, whose kernels are at two
-      // wavefronts per SIMD either way (3D p4 on 16^3 elements 58 against 60 us).
+      // wavefronts per SIMD either way (3D p4 on 16^3 elements 3 % faster so).
       constexpr bool ONE_BY_ONE = !VT::HG;
       T ln_rho[n], ln_t[n];
       const T *sw = fresh(s_w);

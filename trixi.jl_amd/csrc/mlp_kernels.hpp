@@ -1,7 +1,7 @@
 // mlp_kernels.hpp -- the launches of the learned troubled-cell indicator's
 // network (mlp.hpp): parameter packing, inference over a feature matrix,
-// loss gradient, the fixed-order reduction of per-wave gradient rows and
-// Adam. Included by the one translation unit that launches them (the element
+// loss gradient, the fixed-order reduction of its partial rows, one from each
+// workgroup, and Adam. Included by the one translation unit that launches them (the element
 // kernels include only mlp.hpp's device functions).
 #pragma once
 #include "mlp.hpp"
