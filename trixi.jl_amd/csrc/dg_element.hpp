@@ -939,7 +939,8 @@ __device__ __forceinline__ void stage_indicator_2d(const ElemArgs<T> &a, const d
 // which stay in flight until phase B.
 // Minimum wavefronts per SIMD the register allocation must allow: the FP64 3D
 // flux_ranocha variants are held to 168 VGPRs with flux differencing and to 256 with
-// shock capturing, which they meet without scratch memory.
+// shock capturing, which they meet without scratch memory (20 bytes in the p4 stages with
+// boundaries and of two wavefronts per direction).
 template <typename T, int D, int N, int VOL> constexpr int min_waves_per_simd() {
   return sizeof(T) == 8 && D == 3 && VolTraits<VOL>::RAN ? (VOL == VOL_FD_RANOCHA ? 3 : 2) : 1;
 }
