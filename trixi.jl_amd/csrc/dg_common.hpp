@@ -8,7 +8,8 @@
 //   flux                   compressible_euler_3d.jl:420-447 (2D :415-434)
 //   flux_ranocha           compressible_euler_3d.jl:746-793 (2D :686-722), in the
 //                          per-node-logarithm form of the reference's own
-//                          flux_ranocha_turbo kernel (dg_3d_compressible_euler.jl:265-420)
+//                          flux_ranocha_turbo kernel (dg_3d_compressible_euler.jl:265-420);
+//                          FP64 volume lines with the means of log_mean.hpp
 //   ln_mean / inv_ln_mean  src/auxiliary/math.jl:196-263
 //   flux_lax_friedrichs    src/equations/numerical_fluxes.jl:32-45, 166-178, 229-253
 //   max_abs_speed(_naive)  compressible_euler_3d.jl:1112-1177 (2D :1423-1482)

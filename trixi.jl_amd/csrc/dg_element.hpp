@@ -346,10 +346,9 @@ template <int D, int N, int EPB, int O> __device__ __forceinline__ void line_slo
 }
 
 // Surface terms of one line of direction O, added to acc. staged: the tile's
-// states [q][v]. With flux_ranocha and a representation of the node records
-// that holds the sound speed (FP64, and FP32 in the square-root
-// representation), the own face states' primitives and sound speeds come from
-// the records of the two end nodes: wend (read here in FP64).
+// states [q][v]. With flux_ranocha in FP64, and in FP32 in the square-root
+// representation of the node records, the own face states' primitives and sound
+// speeds come from the records of the two end nodes: wend (read here in FP64).
 template <typename T, int D, int N> using LineRecord = std::conditional_t<sizeof(T) == 8, NodeD<D>, NodeR<T, D>>;
 
 // FP64 records: [hr or sqrt(T)][ht][h][hp]. With shock capturing, whose subcell fluxes
